@@ -27,9 +27,10 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t* __restrict__ tr,
         int p = ring_end<F>(8 * lt + q) - 16;
         p = ((p % NBITS) + NBITS) % NBITS;
         const uint32_t w0 = words[sub][(p >> 5) % NW], w1 = words[sub][((p >> 5) + 1) % NW];
-        st[q] = (uint32_t)((((uint64_t)w0 << 32) | w1) >> (48 - (p & 31)));   // bits above 15 are not read
+        st[q] = (uint32_t)((((uint64_t)w0 << 32) | w1) >> (48 - (p & 31))) & 0xffffu;
     }
-    cb_oct(st, w);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = cb_pair(st[2 * q], st[2 * q + 1]);
 #pragma unroll
     for (int q = 0; q < 8; ++q)
     {
