@@ -1,17 +1,11 @@
 // Prefill-size expert products: grouped GEMMs on the MFMA units over EXL3 trellis weights, each weight decoded once per
-// workgroup into LDS in the MFMA operand layout.
-//
-// Work unit = (group of <= 128 dispatch rows of one expert, output columns). One workgroup of 4 waves walks K in steps
-// of 64 (4 tile-rows): every lane decodes one 64-weight strip of a 16 x 16 tile straight from coalesced trellis reads
-// (the decode path's strip mapping: half a wave per tile-row of 8 tiles, four lanes per tile) and stores it as B operand
-// fragments of v_mfma_f32_32x32x16_f16 into one of two LDS stages; after one barrier the 4 waves, arranged 2 (rows) x 2
-// (columns), run the MFMAs of that step with A fragments read from global memory. fp32 accumulation; each output
-// element is one fixed sum (k ascending in MFMA blocks), independent of scheduling.
+// workgroup, straight into the MFMA operand registers of the wave that multiplies it (below, "grouped GEMM"). fp32
+// accumulation; each output element is one fixed sum (k ascending in MFMA blocks), independent of scheduling.
 //
 //   k_pf_prep_tok : rotated gate / up inputs of every dispatch row, xt = RN16(H128(x * suh) * R), token-major
-//   k_pf_gemm<false> : gate or up products of one 256-column block -> fp32 [row][128-block][gate | up][128]
+//   k_pf_gemm<false> : gate or up products of one 512-column block -> fp16 [row][128-block][gate | up][128]
 //   (k_gu_epi)    : fp16 gate / up -> epilogue -> fp16 down-input rows (shared with the decode path)
-//   k_pf_gemm<true>  : down products of one 256-column block -> fp32 [row][128-block][128]
+//   k_pf_gemm<true>  : down products of one 512-column block -> fp32 [row][128-block][128]
 //   (k_dn_combine): rotation * svh, slots summed in slot order (shared with the decode path)
 #include "moe_kernels.hpp"
 
@@ -118,23 +112,14 @@ static dim3 prep_tok_grid(int T, int H)
     return dim3((unsigned)std::max(1L, (units + 15) / 16));
 }
 
-// ---- LDS stages ------------------------------------------------------------------------------------------------------
-// A stage: [row 128 (256 for a pair of groups)][8 chunks of 16 B] = the k-step's 64 inputs of every row; chunk c of row
-//          r sits at slot c ^ ((r >> 1) & 7) of the row, so that the 16 lanes an LDS cycle serves (16 rows, one chunk)
-//          hit 16 different 16-byte bank groups. Copied by the decode waves (each lane 32 B of a row per 16 rows) from
-//          registers loaded two steps ahead.
-// B stage: fragment f = tile-row * 8 + 32-column block (of the 256; of the 128 for a pair), 64 lanes x 16 B; lane L's
-//          16 B at slot f * 64 + bsw(f, L), bsw(f, L) = L ^ ((L >> 4) & 1) ^ ((f & 1) << 3): a bijection on each 16-lane
-//          block (the MFMA reads stay conflict-free) that spreads the 16 lanes of a decode store over 16 bank groups.
-constexpr int PF_A_U4 = 2 * PF_M * 8;
+// ---- B fragments in LDS (mid-size path) -----------------------------------------------------------------------------
+// B stage: fragment f = tile-row * 8 + 32-column block of the 256, 64 lanes x 16 B; lane L's 16 B at slot f * 64 +
+//          bsw(f, L), bsw(f, L) = L ^ ((L >> 4) & 1) ^ ((f & 1) << 3): a bijection on each 16-lane block (the MFMA reads
+//          stay conflict-free) that spreads the 16 lanes of a decode store over 16 bank groups.
 constexpr int PF_B_U4 = 4 * 8 * 64;
-__shared__ u32x4 pf_a0[PF_A_U4];
-__shared__ u32x4 pf_a1[PF_A_U4];
 __shared__ u32x4 pf_b0[PF_B_U4];
 __shared__ u32x4 pf_b1[PF_B_U4];
 
-__device__ __forceinline__ u32x4* a_stage(int s) { return s == 0 ? pf_a0 : pf_a1; }
-__device__ __forceinline__ u32x4* b_stage(int s) { return s == 0 ? pf_b0 : pf_b1; }
 __device__ __forceinline__ int bsw(int f, int L) { return L ^ ((L >> 4) & 1) ^ ((f & 1) << 3); }
 
 // Step barrier: the wave's LDS operations are done (its global loads, register prefetches for later steps, may still be in
@@ -191,364 +176,292 @@ __device__ __forceinline__ void decode_half(const uint32_t (&own)[Fmt<F>::TB / 1
     }
 }
 
-// A quarter strip: stream positions 32 HALF + 16 SUB .. + 15, the same two columns as decode_half<F, HALF> but only
-// input rows 4 SUB .. + 3 and 8 + 4 SUB .. + 3 (dwords 2 SUB, 2 SUB + 1 of each of the column's two fragment slots).
-template <int F, int HALF, int SUB>
-__device__ __forceinline__ void decode_quarter(const uint32_t (&own)[Fmt<F>::TB / 16], u32x4* __restrict__ stage, int kt,
-                                               int col0)
-{
-    constexpr int NW = Fmt<F>::TB / 16;
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int k = 0; k < NW; ++k) asm volatile("" :: "v"(own[k]));
-    const uint32_t prev = __builtin_amdgcn_mov_dpp(own[NW - 1], 0x93, 0xf, 0xf, false);
-    uint32_t fr[2][4];      // [column][dword 2 SUB, 2 SUB + 1 of rows 0-7, then of rows 8-15]
-#pragma unroll
-    for (int j8 = 32 * HALF + 16 * SUB; j8 < 32 * HALF + 16 * SUB + 16; j8 += 8)
-    {
-        uint32_t w[4];
-        oct_weights<F>(prev, own, j8, w);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-        {
-            const int dw = strip_dw(j8 + 2 * q);
-            fr[strip_cidx(j8 + 2 * q) >> 1][((dw >> 2) << 1) + (dw & 1)] = w[q];
-        }
-    }
-#pragma unroll
-    for (int ci = 0; ci < 2; ++ci)
-    {
-        const int col = col0 + lane_col(lane, HALF + 2 * ci);
-        const int f = kt * 8 + (col >> 5);
-        u32x4* fp = stage + f * 64;
-        *reinterpret_cast<u32x2*>(reinterpret_cast<uint32_t*>(fp + bsw(f, col & 31)) + 2 * SUB) = u32x2{fr[ci][0], fr[ci][1]};
-        *reinterpret_cast<u32x2*>(reinterpret_cast<uint32_t*>(fp + bsw(f, (col & 31) + 32)) + 2 * SUB) =
-            u32x2{fr[ci][2], fr[ci][3]};
-    }
-}
-
 // ---- grouped GEMM ----------------------------------------------------------------------------------------------------
-// Work unit: (group of <= 128 rows, matrix, 256-column block); 12 waves, one barrier per k-step (64 k). While waves 0-3
-// run the MFMAs of step i from A / B stage i % 2, waves 4-11 stage step i + 1: they store the A rows loaded two steps
-// earlier and the B fragments decoded from trellis words loaded two steps earlier, and issue the loads of step i + 3.
-// Each SIMD holds one MFMA wave and two decode waves, so the decode (VALU; two waves hide its latency) overlaps the MFMAs.
-//   MFMA wave w: rows 64 (w & 1) .. + 63 (2 row blocks) x columns 128 (w >> 1) .. + 127 (4 column blocks).
-//   decode wave 4 + d: tile-rows 2 (d >> 2) + (lane >> 5), 128-column half (d >> 1) & 1, strip half d & 1; A rows
-//     16 d .. 16 d + 15, 32 B per lane.
-// DOWN = false: gate (matrix 0) or up (1) of the rotated input rows; DOWN = true: down of the down-input rows.
-constexpr int PF_WAVES = 12;
+// Work unit: (group of <= 128 rows, matrix, 512-column block); 8 waves, two per SIMD, all alike. Wave w owns the columns
+// of parity w & 1 (strip half) of 128-column block w >> 1, all rows of the group, and decodes its weights straight into
+// the B operand registers of v_mfma_f32_32x32x16_f16: lane L holds the strip of tile-row L / 32 of a pair of tile-rows
+// (32 k), so an operand's k index 8 (L / 32) + j is input row 8 q + j of that tile-row (q: the strip's upper or lower
+// eight rows), and its column is the lane's strip column. No B fragment passes through the LDS, and no weight is decoded
+// twice in a workgroup. The A rows (128 k at a time) are staged in LDS in operand order and shared by the 8 waves.
+// What bounds it: MFMA (16 per 32 k and wave at 128 rows, 512 cycles) and the decode (115 VALU, 460 cycles) of two waves
+// overlap on a SIMD; the chip then runs into its power limit (the shader clock falls to 1.6-1.8 GHz). Against four MFMA
+// and eight decode waves handing B over through LDS: layer of 8,192 tokens (384 experts, top-6, H 4096, I 2048, K 2 / 3)
+// 5,008 -> 4,427 us, of 517 tokens 1,878 -> 1,433, of 2,048 tokens (H 5120, I 2304, K 2.5 / 2) 3,612 -> 2,959.
+// The scheduling fences keep a pair's operand reads, decode and products apart: the compiler otherwise moves two pairs'
+// decodes together and spills.
+constexpr int PF_WAVES = 8;
+constexpr int PF_KSTEP = 128;                              // k per LDS stage
+constexpr int PF_SUBS = PF_KSTEP / 32;                     // pairs of tile-rows per stage
+constexpr int PF_ST_U4 = PF_M * PF_KSTEP / 8;              // a stage, 16-byte chunks: [sub][q][row block][64 lanes]
+constexpr int PF_COLS = 512;                               // output columns of a unit
+// the products on their way out: rows of 512 columns, padded by 16 bytes (fp16: 128 rows; fp32: 64 rows at a time)
+constexpr int PF_OUT_H = PF_COLS * 2 + 16, PF_OUT_F = PF_COLS * 4 + 16;
+constexpr int PF_LDS = PF_M * PF_OUT_H > 2 * PF_ST_U4 * 16 ? PF_M * PF_OUT_H : 2 * PF_ST_U4 * 16;
+static_assert(PF_OUT_F * PF_M / 2 <= PF_LDS, "half the rows in fp32 fit");
+__shared__ u32x4 pf_lds[PF_LDS / 16];
 
-// cb: the 256-column block of one group's unit; the 128-column block of a pair's (pair = 1)
 struct PfJob {
-    int g, mat, cb, e, r0, nr, K, N, nb128, pair;
+    int g, mat, cb, e, r0, nr, K, N, nb128;
     const bmx_expert* ex;
 };
 
-// An MFMA wave multiplies the 32-row blocks that hold rows of the group (rows past the group's end inside such a block
-// hold copies of its last row) and all its columns (a missing second 128-column half holds stale LDS); neither padding
-// is stored. A wave's tile: MBW 32-row blocks x NBW 32-column blocks (2 x 4 for one group's 128 x 256 tile, 4 x 2 for a
-// pair's 256 x 128), the waves 2 (rows, wave & 1) x 2 (columns, wave >> 1).
-template <int MBW, int NBW>
-struct PfFrag {
-    f16x8 a[MBW];    // [row block]
-    f16x8 b[NBW];    // [column block]
+// Words of a half strip: stream positions 32 HALF .. 32 HALF + 31 of the lane's strip and the 16 bits before them. W0:
+// the first of the strip's words that the half reads (-1: the last word of the strip before it, the ring's wrap included).
+// rows: the tile-rows' address (the same on every lane); strip, prev: the lane's offsets of the strip and of the word
+// before it.
+template <int F, int HALF> struct HalfWords {
+    static constexpr int Q0 = ring_end<F>(32 * HALF) - 16, Q1 = ring_end<F>(32 * HALF + 31);   // first, last + 1 bit
+    static constexpr int W0 = Q0 < 0 ? -1 : Q0 / 32, W1 = (Q1 + 31) / 32, NW = W1 - W0;
+    typedef uint32_t Buf[NW];
 };
 
-// NMB: row blocks of 32 this wave computes (MBW; fewer when the group's rows end inside the wave's blocks)
-template <int MBW, int NBW, int NMB>
-__device__ __forceinline__ void pf_frag_load(PfFrag<MBW, NBW>& f, const u32x4* __restrict__ sa, const u32x4* __restrict__ sb,
-                                             int ks)
+template <int F, int HALF>
+__device__ __forceinline__ void load_half(typename HalfWords<F, HALF>::Buf& w, const uint8_t* rows, uint32_t strip, uint32_t prev)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wm = wave & 1, wn = wave >> 1;
-    const int slot = (2 * ks + (lane >> 5)) ^ ((lane >> 1) & 7);
+    using S = HalfWords<F, HALF>;
 #pragma unroll
-    for (int mb = 0; mb < NMB; ++mb)
-        f.a[mb] = __builtin_bit_cast(f16x8, sa[(32 * MBW * wm + 32 * mb + (lane & 31)) * 8 + slot]);
+    for (int i = 0; i < S::NW; ++i) w[i] = S::W0 + i < 0 ? ldg(rows + prev, 0) : ldg(rows + strip, S::W0 + i);
+}
+
+// The B operands of a half strip: b[ci][q] = the eight input rows 8 q .. + 7 of strip column HALF + 2 ci.
+template <int F, int HALF>
+__device__ __forceinline__ void decode_b(const typename HalfWords<F, HALF>::Buf& w, u32x4 (&b)[2][2])
+{
+    using S = HalfWords<F, HALF>;
+    constexpr RingTab<F> tab;
+    // the words stay allocated until here (a load in flight into a register that is free again would force a wait)
 #pragma unroll
-    for (int nb = 0; nb < NBW; ++nb)
+    for (int k = 0; k < S::NW; ++k) asm volatile("" :: "v"(w[k]));
+    uint32_t own[S::NW];
+#pragma unroll
+    for (int k = 0; k + 1 < S::NW; ++k) own[k] = w[k + 1];
+    own[S::NW - 1] = 0u;
+#pragma unroll
+    for (int j = 32 * HALF; j < 32 * HALF + 32; j += 2)
     {
-        const int fi = ks * 8 + NBW * wn + nb;
-        f.b[nb] = __builtin_bit_cast(f16x8, sb[fi * 64 + bsw(fi, lane)]);
+        // window bit 0 is the first bit of w[0]: strip word W0 (tab.q counts from the word before the strip)
+        const uint32_t v = cb_pair(win_state(w[0], own, tab.q[j] - 32 - 32 * S::W0),
+                                   win_state(w[0], own, tab.q[j + 1] - 32 - 32 * S::W0));
+        b[strip_cidx(j) >> 1][strip_dw(j) >> 2][strip_dw(j) & 3] = v;
     }
 }
 
-template <int MBW, int NBW, int NMB>
-__device__ __forceinline__ void pf_frag_mfma(const PfFrag<MBW, NBW>& f, f32x16 (&acc)[MBW][NBW])
+// A rows of a stage: thread t copies 16-byte chunks (t & 7) and 8 + (t & 7) of rows (t >> 3) and 64 + (t >> 3) (128
+// bytes of a row per 8 lanes). In LDS chunk c = 4 sub + 2 h + q of row r is lane 32 h + r % 32 of operand (sub, q, r /
+// 32); lanes are exchanged by a XOR with 2 (c & 7), which spreads the eight chunks of two rows over the 16 bank groups.
+__device__ __forceinline__ int pf_a_slot(int c, int r)
 {
-#pragma unroll
-    for (int nb = 0; nb < NBW; ++nb)
-#pragma unroll
-        for (int mb = 0; mb < NMB; ++mb)
-            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[mb], f.b[nb], acc[mb][nb], 0, 0, 0);
+    return (((c >> 2) * 2 + (c & 1)) * 4 + (r >> 5)) * 64 + 32 * ((c >> 1) & 1) + ((r & 31) ^ (2 * (c & 7)));
 }
 
-// one k-step of an MFMA wave: 4 sub-steps of 16 k, the fragments of sub-step ks + 1 read while those of ks feed the MFMAs
-template <int MBW, int NBW, int NMB>
-__device__ __forceinline__ void pf_mfma_step(const u32x4* __restrict__ sa, const u32x4* __restrict__ sb,
-                                             f32x16 (&acc)[MBW][NBW])
+template <int NMB>
+struct PfStage {
+    static constexpr int NR = NMB > 2 ? 2 : 1;       // row halves (64 rows) that hold rows of the group
+    u32x4 c[NR][2];
+};
+
+template <int NMB>
+__device__ __forceinline__ void pf_stage_load(PfStage<NMB>& st, const uint16_t* rows, const uint32_t (&off)[2], int k0)
 {
-    PfFrag<MBW, NBW> f0, f1;
-    pf_frag_load<MBW, NBW, NMB>(f0, sa, sb, 0);
-    pf_frag_load<MBW, NBW, NMB>(f1, sa, sb, 1);
-    pf_frag_mfma<MBW, NBW, NMB>(f0, acc);
-    pf_frag_load<MBW, NBW, NMB>(f0, sa, sb, 2);
-    pf_frag_mfma<MBW, NBW, NMB>(f1, acc);
-    pf_frag_load<MBW, NBW, NMB>(f1, sa, sb, 3);
-    pf_frag_mfma<MBW, NBW, NMB>(f0, acc);
-    pf_frag_mfma<MBW, NBW, NMB>(f1, acc);
+    const char* p = reinterpret_cast<const char*>(rows + k0);
+#pragma unroll
+    for (int j = 0; j < PfStage<NMB>::NR; ++j)
+    {
+        st.c[j][0] = ldg4(p + off[j]);
+        st.c[j][1] = ldg4(p + off[j] + 128);
+    }
 }
 
-// the MFMA loop over K (one barrier per step, as the decode waves)
-template <int MBW, int NBW, int NMB>
-__device__ __forceinline__ void pf_mfma_loop(int KT, f32x16 (&acc)[MBW][NBW])
+template <int NMB>
+__device__ __forceinline__ void pf_stage_store(const PfStage<NMB>& st, u32x4* __restrict__ lds)
 {
+    const int r = threadIdx.x >> 3, c = threadIdx.x & 7;
+#pragma unroll
+    for (int j = 0; j < PfStage<NMB>::NR; ++j)
+    {
+        lds[pf_a_slot(c, r + 64 * j)] = st.c[j][0];
+        lds[pf_a_slot(c + 8, r + 64 * j)] = st.c[j][1];
+    }
+}
+
+// The unit's k-loop of one wave, NMB 32-row blocks: per stage of 128 k, 4 pairs of tile-rows. The words of a pair are
+// requested four pairs ahead (each register set again right after its use), the A rows one stage ahead; one barrier per
+// stage. WORK false: a wave without columns (past the matrix's last block), which only copies A rows.
+template <int F, int HALF, int NMB, bool WORK>
+__device__ __forceinline__ void pf_loop(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc, int cbo,
+                                        f32x16 (&acc)[2][NMB])
+{
+    constexpr int TB = Fmt<F>::TB;
+    using S = HalfWords<F, HALF>;
+    const int lane = threadIdx.x & 63, h = lane >> 5, t = (lane >> 2) & 7, s = lane & 3;
+    const uint32_t row_bytes = (uint32_t)(jb.N / 16) * TB;
+    // offsets from wave-uniform addresses; the word before a strip is the tile's last one for its first strip
+    const uint32_t strip = (uint32_t)h * row_bytes + (uint32_t)(cbo * 8 + t) * TB + (uint32_t)s * (TB / 4);
+    const uint32_t prev = s ? strip - 4 : strip + TB - 4;
+    const int KT = jb.K / PF_KSTEP;
+    const uint16_t* rows = asrc + (size_t)jb.r0 * jb.K;
+    uint32_t aoff[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        aoff[j] = 2u * ((uint32_t)min((int)(threadIdx.x >> 3) + 64 * j, jb.nr - 1) * (uint32_t)jb.K + 8u * (threadIdx.x & 7));
+    PfStage<NMB> st;
+    typename S::Buf w[PF_SUBS];
+    pf_stage_load<NMB>(st, rows, aoff, 0);
+    if (WORK)
+    {
+#pragma unroll
+        for (int j = 0; j < PF_SUBS; ++j) load_half<F, HALF>(w[j], mat_base + (size_t)(2 * j) * row_bytes, strip, prev);
+    }
+    pf_stage_store<NMB>(st, pf_lds);
+    step_barrier();
     for (int i = 0; i < KT; ++i)
     {
-        pf_mfma_step<MBW, NBW, NMB>(a_stage(i & 1), b_stage(i & 1), acc);
+        const int in = min(i + 1, KT - 1);          // past the last stage: its own loads again, never used
+        const u32x4* lds = pf_lds + (i & 1) * PF_ST_U4;
+        pf_stage_load<NMB>(st, rows, aoff, in * PF_KSTEP);
+        if (WORK)
+        {
+            const uint8_t* pn = mat_base + (size_t)(2 * PF_SUBS) * in * row_bytes;
+#pragma unroll
+            for (int j = 0; j < PF_SUBS; ++j)
+            {
+                f16x8 a[2][NMB];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int m = 0; m < NMB; ++m)
+                        a[q][m] = __builtin_bit_cast(f16x8, lds[((2 * j + q) * 4 + m) * 64 + 32 * h +
+                                                                ((lane & 31) ^ (2 * (4 * (j & 1) + 2 * h + q)))]);
+                __builtin_amdgcn_sched_barrier(0);
+                u32x4 b[2][2];
+                decode_b<F, HALF>(w[j], b);
+                __builtin_amdgcn_sched_barrier(0);
+                load_half<F, HALF>(w[j], pn + (size_t)(2 * j) * row_bytes, strip, prev);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+                        for (int m = 0; m < NMB; ++m)
+                            acc[ci][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                a[q][m], __builtin_bit_cast(f16x8, b[ci][q]), acc[ci][m], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        pf_stage_store<NMB>(st, pf_lds + ((i + 1) & 1) * PF_ST_U4);
         step_barrier();
     }
 }
 
-// A rows of one k-step: lane's 32 bytes (chunks 2 (lane & 3), + 1) of row 16 d + (lane >> 2)
-struct PfArow {
-    u32x4 c[2];
-};
-
-__device__ __forceinline__ void a_fetch(PfArow& r, const uint16_t* rowp, int k0)
+// The unit's products out of the accumulators, through LDS (the A stages are done with) so that whole rows of the unit's
+// columns are stored 16 bytes per lane: accumulator element v of lane L is row 8 (v / 4) + 4 (L / 32) + v % 4 of its row
+// block, column lane_col(L, HALF + 2 ci) of the wave's 128-column block. Gate / up products are stored as fp16 (the value
+// the epilogue would round them to), down products as fp32, 64 rows at a time.
+template <bool DOWN, int NMB>
+__device__ __forceinline__ void pf_out(const GvArgs& a, const PfJob& jb, const f32x16 (&acc)[2][NMB])
 {
-    const int lane = threadIdx.x & 63;
-    const uint16_t* p = rowp + k0 + 16 * (lane & 3);
-    r.c[0] = ldg4(p);
-    r.c[1] = ldg4(p + 8);
-}
-
-__device__ __forceinline__ void a_store(const PfArow& r, u32x4* __restrict__ stage, int row)
-{
-    const int lane = threadIdx.x & 63, x = (row >> 1) & 7;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    char* lds = reinterpret_cast<char*>(pf_lds);
+    constexpr int RB = DOWN ? 2 : NMB;                                // row blocks per round
+    constexpr int ES = DOWN ? 4 : 2, RS = DOWN ? PF_OUT_F : PF_OUT_H;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) stage[row * 8 + ((2 * (lane & 3) + j) ^ x)] = r.c[j];
-}
-
-// The loop is straight-line code (every step issues the same loads, past-the-end steps re-read the last one, a missing
-// second 128-column half decodes the first one's tiles again), so the compiler's wait counts for the prefetched
-// registers stay exact and the waits land only where the data is two steps old.
-// One group (PAIR false): decode wave 4 + d decodes strip half d & 1 of 128-column half (d >> 1) & 1 and copies A rows
-// 16 d .. + 15. A pair (PAIR true, one 128-column block): strip quarter 2 HALF + SUB = d & 3, A rows 32 d .. + 31.
-template <int F, int HALF, int SUB, bool PAIR, bool ACOPY>
-__device__ __forceinline__ void pf_decoder(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc, int d)
-{
-    constexpr int TB = Fmt<F>::TB, NW = TB / 16, NA = PAIR ? 2 : 1;
-    const int lane = threadIdx.x & 63;
-    const int h = lane >> 5, t = (lane >> 2) & 7, s = lane & 3;
-    const int kt = 2 * (d >> 2) + h, th = (d >> 1) & 1;
-    const int tcol = PAIR ? jb.cb : min(2 * jb.cb + th, jb.nb128 - 1);
-    const size_t row_bytes = (size_t)(jb.N / 16) * TB, step_bytes = 4 * row_bytes;
-    const uint8_t* p = mat_base + (size_t)kt * row_bytes + (size_t)(tcol * 8 + t) * TB + s * (TB / 4);
-    const int KT = jb.K / 64;
-    // this lane's A rows (rows past the group's end read its last row; their products are not stored)
-    int arow[NA];
-    const uint16_t* rowp[NA];
-#pragma unroll
-    for (int j = 0; j < NA; ++j)
+    for (int m0 = 0; m0 < NMB; m0 += RB)
     {
-        arow[j] = 16 * NA * d + 16 * j + (lane >> 2);
-        rowp[j] = asrc + (size_t)(jb.r0 + min(arow[j], jb.nr - 1)) * jb.K;
-    }
-    auto wp = [&](int step) { return p + (size_t)min(step, KT - 1) * step_bytes; };
-    auto ak = [&](int step) { return 64 * min(step, KT - 1); };
-    auto dec = [&](const uint32_t (&w)[NW], u32x4* stage) {
-        if constexpr (PAIR) decode_quarter<F, HALF, SUB>(w, stage, kt, 0);
-        else decode_half<F, HALF>(w, stage, kt, 128 * th, threadIdx.x & 63);
-    };
-    auto fetch = [&](PfArow (&a)[NA], int step) {
+        if (m0) step_barrier();                                       // the round before is read out
 #pragma unroll
-        for (int j = 0; j < NA; ++j) a_fetch(a[j], rowp[j], ak(step));
-    };
-    auto store = [&](const PfArow (&a)[NA], u32x4* stage) {
+        for (int m = m0; m < NMB && m < m0 + RB; ++m)
 #pragma unroll
-        for (int j = 0; j < NA; ++j) a_store(a[j], stage, arow[j]);
-    };
-    // DEPTH register sets (words and A rows) in rotation: step s is loaded into set s % DEPTH DEPTH - 1 steps before it
-    // is staged. The MFMA waves set the kernel's register count; a group's decoder has the room for a fourth set up to
-    // K 3 (six words a strip), a pair's (twice the A rows) or a K 4 one's (eight words) keeps three.
-    constexpr int DEPTH = (PAIR || NW > 6) ? 3 : 4;
-    uint32_t w[DEPTH][NW];
-    PfArow ar[DEPTH][NA];
+            for (int ci = 0; ci < 2; ++ci)
 #pragma unroll
-    for (int q = 0; q < DEPTH; ++q)
-    {
-        if (ACOPY) fetch(ar[q], q);
-        load_words<false>(w[q], wp(q));
-    }
-    dec(w[0], pf_b0);
-    if (ACOPY) store(ar[0], pf_a0);
-    step_barrier();
-    // sub-step q of the trip from step i: load step i + q + DEPTH into set q (staged in the sub-step before), stage step
-    // i + q + 1 from set (q + 1) % DEPTH into stage (i + q + 1) % 2
-    for (int i = 0; i < KT; i += DEPTH)
-    {
-#pragma unroll
-        for (int q = 0; q < DEPTH; ++q)
+                for (int v = 0; v < 16; ++v)
+                {
+                    const int row = 32 * (m - m0) + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                    const int col = 128 * (wave >> 1) + lane_col(lane, (wave & 1) + 2 * ci);
+                    char* p = lds + row * RS + col * ES;
+                    if (DOWN) *reinterpret_cast<float*>(p) = acc[ci][m][v];
+                    else *reinterpret_cast<uint16_t*>(p) = f2h_r(0.0f + acc[ci][m][v]);
+                }
+        step_barrier();
+        // 16-byte pieces: PPR per row; piece q of a row is in 128-column block q / PPB
+        constexpr int PPR = PF_COLS * ES / 16, PPB = PPR / 4;
+        const int rows = min(jb.nr - 32 * m0, 32 * RB);
+        for (int i = threadIdx.x; i < rows * PPR; i += PF_WAVES * 64)
         {
-            if (ACOPY) fetch(ar[q], i + q + DEPTH);
-            load_words<false>(w[q], wp(i + q + DEPTH));
-            dec(w[(q + 1) % DEPTH], b_stage((i + q + 1) & 1));
-            if (ACOPY) store(ar[(q + 1) % DEPTH], a_stage((i + q + 1) & 1));
-            step_barrier();
-            if (i + q + 1 >= KT) return;
+            const int row = i / PPR, q = i % PPR, cbo = 4 * jb.cb + q / PPB;
+            if (cbo >= jb.nb128) continue;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(lds + row * RS + q * 16);
+            const size_t r = (size_t)(jb.r0 + 32 * m0 + row);
+            char* out = DOWN ? reinterpret_cast<char*>(a.part_dn + (r * a.NBH + cbo) * 128)
+                             : reinterpret_cast<char*>(reinterpret_cast<uint16_t*>(a.part_gu) + (r * a.NB + cbo) * 256 +
+                                                       jb.mat * 128);
+            *reinterpret_cast<u32x4*>(out + (q % PPB) * 16) = v;
         }
     }
 }
 
-// A rows are copied only where an MFMA wave reads them: the 32-row blocks that hold rows of the group
-template <int F, bool PAIR>
-__device__ __forceinline__ void pf_decoder_role(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc, int d)
+template <bool DOWN, int F, int HALF, int NMB>
+__device__ __forceinline__ void pf_unit(const GvArgs& a, const PfJob& jb, const uint8_t* base, const uint16_t* asrc, int cbo)
 {
-    const bool acopy = (PAIR ? 32 : 16) * d < (jb.nr + 31) / 32 * 32;
-    if (PAIR)
+    f32x16 acc[2][NMB];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NMB; ++j) acc[i][j] = f32x16{};
+    if (cbo < jb.nb128) pf_loop<F, HALF, NMB, true>(jb, base, asrc, cbo, acc);
+    else pf_loop<F, HALF, NMB, false>(jb, base, asrc, cbo, acc);
+    pf_out<DOWN, NMB>(a, jb, acc);
+}
+
+template <bool DOWN, int F, int HALF>
+__device__ __forceinline__ void pf_unit_rows(const GvArgs& a, const PfJob& jb, const uint8_t* base, const uint16_t* asrc,
+                                             int cbo)
+{
+    switch ((jb.nr + 31) / 32)
     {
-        // quarter d & 3 (a switch on a wave-uniform value: one path per wave)
-        switch ((d & 3) + (acopy ? 4 : 0))
-        {
-            case 0: pf_decoder<F, 0, 0, true, false>(jb, mat_base, asrc, d); break;
-            case 1: pf_decoder<F, 0, 1, true, false>(jb, mat_base, asrc, d); break;
-            case 2: pf_decoder<F, 1, 0, true, false>(jb, mat_base, asrc, d); break;
-            case 3: pf_decoder<F, 1, 1, true, false>(jb, mat_base, asrc, d); break;
-            case 4: pf_decoder<F, 0, 0, true, true>(jb, mat_base, asrc, d); break;
-            case 5: pf_decoder<F, 0, 1, true, true>(jb, mat_base, asrc, d); break;
-            case 6: pf_decoder<F, 1, 0, true, true>(jb, mat_base, asrc, d); break;
-            default: pf_decoder<F, 1, 1, true, true>(jb, mat_base, asrc, d); break;
-        }
-    }
-    else if (acopy)
-    {
-        if (d & 1) pf_decoder<F, 1, 0, false, true>(jb, mat_base, asrc, d);
-        else pf_decoder<F, 0, 0, false, true>(jb, mat_base, asrc, d);
-    }
-    else
-    {
-        if (d & 1) pf_decoder<F, 1, 0, false, false>(jb, mat_base, asrc, d);
-        else pf_decoder<F, 0, 0, false, false>(jb, mat_base, asrc, d);
+        case 1: pf_unit<DOWN, F, HALF, 1>(a, jb, base, asrc, cbo); break;
+        case 2: pf_unit<DOWN, F, HALF, 2>(a, jb, base, asrc, cbo); break;
+        case 3: pf_unit<DOWN, F, HALF, 3>(a, jb, base, asrc, cbo); break;
+        default: pf_unit<DOWN, F, HALF, 4>(a, jb, base, asrc, cbo); break;
     }
 }
 
-template <int F>
-__device__ __forceinline__ void pf_decoder_any(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc)
+template <bool DOWN, int F>
+__device__ __forceinline__ void pf_unit_half(const GvArgs& a, const PfJob& jb, const uint8_t* base, const uint16_t* asrc,
+                                             int wave)
 {
-    const int d = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) - 4);
-    if (jb.pair) pf_decoder_role<F, true>(jb, mat_base, asrc, d);
-    else pf_decoder_role<F, false>(jb, mat_base, asrc, d);
-}
-
-// Store of an MFMA wave's products: accumulator element v of lane L is row 8 (v / 4) + 4 (L / 32) + v % 4, column L % 32
-// of its 32 x 32 block; rows past the group's end are not stored.
-template <bool DOWN, int MBW, int NBW>
-__device__ __forceinline__ void pf_store(const GvArgs& a, const PfJob& jb, const f32x16 (&acc)[MBW][NBW])
-{
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wm = wave & 1, wn = wave >> 1;
-    // the wave's 128-column output block and its first column in it
-    const int cbo = jb.pair ? jb.cb : 2 * jb.cb + wn, c0 = jb.pair ? 32 * NBW * wn : 0;
-    if (cbo >= jb.nb128) return;
-#pragma unroll
-    for (int mb = 0; mb < MBW; ++mb)
-    {
-        if (32 * MBW * wm + 32 * mb >= jb.nr) continue;
-#pragma unroll
-        for (int nb = 0; nb < NBW; ++nb)
-        {
-            const int col = c0 + 32 * nb + (lane & 31);
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
-            {
-                const int row = 32 * MBW * wm + 32 * mb + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (row >= jb.nr) continue;
-                const size_t r = (size_t)(jb.r0 + row);
-                if (DOWN) a.part_dn[(r * a.NBH + cbo) * 128 + col] = acc[mb][nb][v];
-                else
-                    reinterpret_cast<uint16_t*>(a.part_gu)[(r * a.NB + cbo) * 256 + jb.mat * 128 + col] =
-                        f2h_r(0.0f + acc[mb][nb][v]);
-            }
-        }
-    }
-}
-
-// The MFMA waves of one tile shape: row blocks past the group's end are neither read nor multiplied (a wave with none
-// only keeps the barriers).
-template <bool DOWN, int MBW, int NBW>
-__device__ __forceinline__ void pf_mfma_wave(const GvArgs& a, const PfJob& jb, int KT)
-{
-    const int wm = (threadIdx.x >> 6) & 1;
-    f32x16 acc[MBW][NBW];
-#pragma unroll
-    for (int i = 0; i < MBW; ++i)
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) acc[i][j] = f32x16{};
-    const int nmb = min(MBW, max(0, (jb.nr - 32 * MBW * wm + 31) / 32));
-    step_barrier();
-    switch (nmb)
-    {
-        case 0: for (int i = 0; i < KT; ++i) step_barrier(); break;
-        case 1: pf_mfma_loop<MBW, NBW, 1>(KT, acc); break;
-        case 2: pf_mfma_loop<MBW, NBW, 2>(KT, acc); break;
-        case 3: if constexpr (MBW >= 3) pf_mfma_loop<MBW, NBW, 3>(KT, acc); break;
-        default: if constexpr (MBW >= 4) pf_mfma_loop<MBW, NBW, 4>(KT, acc); break;
-    }
-    pf_store<DOWN, MBW, NBW>(a, jb, acc);
+    const int cbo = 4 * jb.cb + (wave >> 1);
+    if (wave & 1) pf_unit_rows<DOWN, F, 1>(a, jb, base, asrc, cbo);
+    else pf_unit_rows<DOWN, F, 0>(a, jb, base, asrc, cbo);
 }
 
 template <bool DOWN>
-__global__ __launch_bounds__(PF_WAVES * 64) void k_pf_gemm(GvArgs a)
+__global__ __launch_bounds__(PF_WAVES * 64, 2) void k_pf_gemm(GvArgs a)
 {
     const int nb128 = DOWN ? a.NBH : a.NB;     // 128-column blocks of the output
-    const int NB2 = (nb128 + 1) / 2;
+    const int NB4 = (nb128 + 3) / 4;
     const int lid = xcd_block(blockIdx.x, gridDim.x);
     PfJob jb;
     jb.nb128 = nb128;
-    if (DOWN) { jb.g = lid / NB2; jb.mat = 2; jb.cb = lid % NB2; }
-    else { jb.g = lid / (2 * NB2); jb.mat = (lid / NB2) & 1; jb.cb = lid % NB2; }
+    if (DOWN) { jb.g = lid / NB4; jb.mat = 2; jb.cb = lid % NB4; }
+    else { jb.g = lid / (2 * NB4); jb.mat = (lid / NB4) & 1; jb.cb = lid % NB4; }
     if (jb.g >= *a.ngroups) return;
     jb.e = a.groups[3 * jb.g];
     if (group_skipped(a, jb.e)) return;
     jb.r0 = a.groups[3 * jb.g + 1];
     jb.nr = a.groups[3 * jb.g + 2];
-    jb.pair = 0;
-    if (a.pf_pairs)
-    {
-        // groups 2 j and 2 j + 1 of an expert (consecutive rows) form a pair; its units are both groups' units, unit
-        // (group 2 j + q, 256-column block c) taking 128-column block 2 c + q of all the pair's rows
-        const int base = a.offsets[jb.e], cnt = a.offsets[jb.e + 1] - base;
-        const int q = (jb.r0 - base) / PF_M, ng = (cnt + PF_M - 1) / PF_M;
-        if ((q & 1) || q + 1 < ng)
-        {
-            const int q0 = q & ~1;
-            jb.pair = 1;
-            jb.r0 = base + q0 * PF_M;
-            jb.nr = min(2 * PF_M, cnt - q0 * PF_M);
-            jb.cb = 2 * jb.cb + (q & 1);
-            if (jb.cb >= nb128) return;        // an odd block count: the last 256-column block has one half
-        }
-    }
     jb.ex = jb.e == a.E ? a.shared : a.experts + jb.e;
     jb.K = DOWN ? a.I : a.H;
     jb.N = DOWN ? a.H : a.I;
-    const int wave = threadIdx.x >> 6;
-    const int KT = jb.K / 64;
-
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint16_t* asrc = DOWN ? a.act_rows : a.xt + (size_t)jb.mat * a.R_max * a.H;
-    if (wave >= 4)
+    const uint8_t* base = reinterpret_cast<const uint8_t*>(jb.ex->tr[jb.mat]);
+    switch (jb.ex->fmt[jb.mat])
     {
-        const uint8_t* base = reinterpret_cast<const uint8_t*>(jb.ex->tr[jb.mat]);
-        switch (jb.ex->fmt[jb.mat])
-        {
-            case BMX_TF_K2: pf_decoder_any<BMX_TF_K2>(jb, base, asrc); break;
-            case BMX_TF_K25: pf_decoder_any<BMX_TF_K25>(jb, base, asrc); break;
-            case BMX_TF_K3: pf_decoder_any<BMX_TF_K3>(jb, base, asrc); break;
-            default: pf_decoder_any<BMX_TF_K4>(jb, base, asrc); break;
-        }
-        return;
+        case BMX_TF_K2: pf_unit_half<DOWN, BMX_TF_K2>(a, jb, base, asrc, wave); break;
+        case BMX_TF_K25: pf_unit_half<DOWN, BMX_TF_K25>(a, jb, base, asrc, wave); break;
+        case BMX_TF_K3: pf_unit_half<DOWN, BMX_TF_K3>(a, jb, base, asrc, wave); break;
+        default: pf_unit_half<DOWN, BMX_TF_K4>(a, jb, base, asrc, wave); break;
     }
-    if (jb.pair) pf_mfma_wave<DOWN, 4, 2>(a, jb, KT);
-    else pf_mfma_wave<DOWN, 2, 4>(a, jb, KT);
 }
 
 // ---- mid-size grouped GEMM: groups of <= 32 rows, every wave decodes and multiplies ------------------------------------
@@ -765,13 +678,6 @@ static PrefillPlan prefill_plan(const MoeShape& m)
 
 int prefill_rows_per_group() { return PF_M; }
 
-// BMX_PF_PAIRS=0: every group its own 128-row tile (the products are the same bits either way)
-static bool prefill_pairs_allowed()
-{
-    const char* v = getenv("BMX_PF_PAIRS");
-    return !(v && *v == '0');
-}
-
 // BMX_PF_FAST_ACT=0: the prefill path's epilogue keeps the fixed-sequence activation of the decode path
 static bool prefill_fast_act()
 {
@@ -950,7 +856,6 @@ int launch_prefill_experts(const MoeShape& m, const void* x, const bmx_routes* r
     a.filter = 0;
     a.act_in_down = 0;
     a.gu_half = 1;
-    a.pf_pairs = prefill_pairs_allowed() ? 1 : 0;
     a.fast_act = prefill_fast_act() ? 1 : 0;
     int rc = BMX_OK;
     if (stages & (1 << BMX_STAGE_PREP))
@@ -961,7 +866,7 @@ int launch_prefill_experts(const MoeShape& m, const void* x, const bmx_routes* r
         if (!(stages & (1 << st))) continue;
         GvArgs b = a;
         b.filter = f;
-        hipLaunchKernelGGL(k_pf_gemm<false>, dim3((unsigned)(p.G_max * 2 * ((p.NB + 1) / 2))), dim3(PF_WAVES * 64), 0, s, b);
+        hipLaunchKernelGGL(k_pf_gemm<false>, dim3((unsigned)(p.G_max * 2 * ((p.NB + 3) / 4))), dim3(PF_WAVES * 64), 0, s, b);
     }
     if (stages & (1 << BMX_STAGE_ACT)) rc = launch_epilogue(a, BMX_STAGE_ACT, s);
     for (int f = 0; f < 3 && !rc; ++f)
@@ -970,7 +875,7 @@ int launch_prefill_experts(const MoeShape& m, const void* x, const bmx_routes* r
         if (!(stages & (1 << st))) continue;
         GvArgs b = a;
         b.filter = f;
-        hipLaunchKernelGGL(k_pf_gemm<true>, dim3((unsigned)(p.G_max * ((p.NBH + 1) / 2))), dim3(PF_WAVES * 64), 0, s, b);
+        hipLaunchKernelGGL(k_pf_gemm<true>, dim3((unsigned)(p.G_max * ((p.NBH + 3) / 4))), dim3(PF_WAVES * 64), 0, s, b);
     }
     if (!rc && (stages & (1 << BMX_STAGE_COMBINE))) rc = launch_epilogue(a, BMX_STAGE_COMBINE, s);
     if (!rc && (stages & (1 << BMX_STAGE_DOWN_OUT))) rc = launch_epilogue(a, BMX_STAGE_DOWN_OUT, s);
