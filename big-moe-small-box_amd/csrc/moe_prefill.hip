@@ -223,27 +223,26 @@ __device__ __forceinline__ void load_half(typename HalfWords<F, HALF>::Buf& w, c
     for (int i = 0; i < S::NW; ++i) w[i] = S::W0 + i < 0 ? ldg(rows + prev, 0) : ldg(rows + strip, S::W0 + i);
 }
 
-// The B operands of a half strip: b[ci][q] = the eight input rows 8 q .. + 7 of strip column HALF + 2 ci.
-template <int F, int HALF>
-__device__ __forceinline__ void decode_b(const typename HalfWords<F, HALF>::Buf& w, u32x4 (&b)[2][2])
+// B operand (CI, Q) of a half strip: the eight input rows 8 Q .. + 7 of strip column HALF + 2 CI, four pairs of weights.
+template <int F, int HALF, int CI, int Q>
+__device__ __forceinline__ u32x4 decode_b(const typename HalfWords<F, HALF>::Buf& w)
 {
     using S = HalfWords<F, HALF>;
     constexpr RingTab<F> tab;
-    // the words stay allocated until here (a load in flight into a register that is free again would force a wait)
-#pragma unroll
-    for (int k = 0; k < S::NW; ++k) asm volatile("" :: "v"(w[k]));
     uint32_t own[S::NW];
 #pragma unroll
     for (int k = 0; k + 1 < S::NW; ++k) own[k] = w[k + 1];
     own[S::NW - 1] = 0u;
+    u32x4 b;
 #pragma unroll
-    for (int j = 32 * HALF; j < 32 * HALF + 32; j += 2)
+    for (int g = 0; g < 4; ++g)
     {
+        const int j = 32 * HALF + 8 * g + 4 * CI + 2 * Q;      // strip_cidx(j) = HALF + 2 CI, strip_dw(j) = g + 4 Q
         // window bit 0 is the first bit of w[0]: strip word W0 (tab.q counts from the word before the strip)
-        const uint32_t v = cb_pair(win_state(w[0], own, tab.q[j] - 32 - 32 * S::W0),
-                                   win_state(w[0], own, tab.q[j + 1] - 32 - 32 * S::W0));
-        b[strip_cidx(j) >> 1][strip_dw(j) >> 2][strip_dw(j) & 3] = v;
+        b[g] = cb_pair(win_state(w[0], own, tab.q[j] - 32 - 32 * S::W0),
+                       win_state(w[0], own, tab.q[j + 1] - 32 - 32 * S::W0));
     }
+    return b;
 }
 
 // A rows of a stage: thread t copies 16-byte chunks (t & 7) and 8 + (t & 7) of rows (t >> 3) and 64 + (t >> 3) (128
@@ -284,6 +283,39 @@ __device__ __forceinline__ void pf_stage_store(const PfStage<NMB>& st, u32x4* __
     }
 }
 
+// One operand slot of a wave: operand (CI, Q) of the words w is decoded into b while the products of the operand before
+// it (bp, columns 1 - CI, rows ap) run, one MFMA per 29 / NMB VALU instructions: the two waves of a SIMD march in step
+// from barrier to barrier, so an MFMA burst and a decode burst would each leave the other unit idle.
+template <int F, int HALF, int CI, int Q, int NMB>
+__device__ __forceinline__ void pf_slot(const typename HalfWords<F, HALF>::Buf& w, u32x4& b, const u32x4& bp,
+                                        const f16x8 (&ap)[NMB], f32x16 (&acc)[2][NMB])
+{
+    b = decode_b<F, HALF, CI, Q>(w);
+#pragma unroll
+        for (int m = 0; m < NMB; ++m)
+            acc[1 - CI][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ap[m], __builtin_bit_cast(f16x8, bp), acc[1 - CI][m],
+                                                                    0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < NMB; ++m)
+        {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);            // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x2, 28 / NMB, 0);     // VALU
+        }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The A operands (q) of pair j of a stage
+template <int NMB>
+__device__ __forceinline__ void pf_a_read(f16x8 (&a)[NMB], const u32x4* __restrict__ lds, int j, int q)
+{
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+#pragma unroll
+    for (int m = 0; m < NMB; ++m)
+        a[m] = __builtin_bit_cast(f16x8, lds[((2 * j + q) * 4 + m) * 64 + 32 * h +
+                                             ((lane & 31) ^ (2 * (4 * (j & 1) + 2 * h + q)))]);
+    __builtin_amdgcn_sched_barrier(0);        // read a slot ahead of their use
+}
+
 // The unit's k-loop of one wave, NMB 32-row blocks: per stage of 128 k, 4 pairs of tile-rows. The words of a pair are
 // requested four pairs ahead (each register set again right after its use), the A rows one stage ahead; one barrier per
 // stage. WORK false: a wave without columns (past the matrix's last block), which only copies A rows.
@@ -306,11 +338,17 @@ __device__ __forceinline__ void pf_loop(const PfJob& jb, const uint8_t* mat_base
         aoff[j] = 2u * ((uint32_t)min((int)(threadIdx.x >> 3) + 64 * j, jb.nr - 1) * (uint32_t)jb.K + 8u * (threadIdx.x & 7));
     PfStage<NMB> st;
     typename S::Buf w[PF_SUBS];
+    u32x4 b0, b1;
+    f16x8 a0[NMB], a1[NMB];
     pf_stage_load<NMB>(st, rows, aoff, 0);
     if (WORK)
     {
 #pragma unroll
         for (int j = 0; j < PF_SUBS; ++j) load_half<F, HALF>(w[j], mat_base + (size_t)(2 * j) * row_bytes, strip, prev);
+        // the pipeline starts with an operand of zeros (its products add nothing)
+        b1 = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int m = 0; m < NMB; ++m) a1[m] = f16x8{};
     }
     pf_stage_store<NMB>(st, pf_lds);
     step_barrier();
@@ -325,32 +363,26 @@ __device__ __forceinline__ void pf_loop(const PfJob& jb, const uint8_t* mat_base
 #pragma unroll
             for (int j = 0; j < PF_SUBS; ++j)
             {
-                f16x8 a[2][NMB];
+                // the words stay allocated until here (a load in flight into a register that is free again would force
+                // a wait)
 #pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int m = 0; m < NMB; ++m)
-                        a[q][m] = __builtin_bit_cast(f16x8, lds[((2 * j + q) * 4 + m) * 64 + 32 * h +
-                                                                ((lane & 31) ^ (2 * (4 * (j & 1) + 2 * h + q)))]);
-                __builtin_amdgcn_sched_barrier(0);
-                u32x4 b[2][2];
-                decode_b<F, HALF>(w[j], b);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int k = 0; k < S::NW; ++k) asm volatile("" :: "v"(w[j][k]));
+                pf_a_read<NMB>(a0, lds, j, 0);
+                pf_slot<F, HALF, 0, 0, NMB>(w[j], b0, b1, a1, acc);
+                pf_slot<F, HALF, 1, 0, NMB>(w[j], b1, b0, a0, acc);
+                pf_a_read<NMB>(a1, lds, j, 1);
+                pf_slot<F, HALF, 0, 1, NMB>(w[j], b0, b1, a0, acc);
+                pf_slot<F, HALF, 1, 1, NMB>(w[j], b1, b0, a1, acc);
                 load_half<F, HALF>(w[j], pn + (size_t)(2 * j) * row_bytes, strip, prev);
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int ci = 0; ci < 2; ++ci)
-#pragma unroll
-                        for (int m = 0; m < NMB; ++m)
-                            acc[ci][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                a[q][m], __builtin_bit_cast(f16x8, b[ci][q]), acc[ci][m], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
             }
         }
         pf_stage_store<NMB>(st, pf_lds + ((i + 1) & 1) * PF_ST_U4);
         step_barrier();
     }
+    if (WORK)
+#pragma unroll
+        for (int m = 0; m < NMB; ++m)
+            acc[1][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[m], __builtin_bit_cast(f16x8, b1), acc[1][m], 0, 0, 0);
 }
 
 // The unit's products out of the accumulators, through LDS (the A stages are done with) so that whole rows of the unit's
