@@ -189,12 +189,12 @@ __device__ __forceinline__ void decode_half(const uint32_t (&own)[Fmt<F>::TB / 1
 // 5,008 -> 4,427 us, of 517 tokens 1,878 -> 1,433, of 2,048 tokens (H 5120, I 2304, K 2.5 / 2) 3,612 -> 2,959.
 // The scheduling fences keep a pair's operand reads, decode and products apart: the compiler otherwise moves two pairs'
 // decodes together and spills.
-constexpr int PF_WAVES = 8;
-constexpr int PF_KSTEP = 128;                              // k per LDS stage
+constexpr int PF_WAVES = 4;
+constexpr int PF_KSTEP = 64;                               // k per LDS stage
 constexpr int PF_SUBS = PF_KSTEP / 32;                     // pairs of tile-rows per stage
 constexpr int PF_ST_U4 = PF_M * PF_KSTEP / 8;              // a stage, 16-byte chunks: [sub][q][row block][64 lanes]
-constexpr int PF_COLS = 512;                               // output columns of a unit
-// the products on their way out: rows of 512 columns, padded by 16 bytes (fp16: 128 rows; fp32: 64 rows at a time)
+constexpr int PF_COLS = 256;                               // output columns of a unit
+// the products on their way out: rows of 256 columns, padded by 16 bytes (fp16: 128 rows; fp32: 64 rows at a time)
 constexpr int PF_OUT_H = PF_COLS * 2 + 16, PF_OUT_F = PF_COLS * 4 + 16;
 constexpr int PF_LDS = PF_M * PF_OUT_H > 2 * PF_ST_U4 * 16 ? PF_M * PF_OUT_H : 2 * PF_ST_U4 * 16;
 static_assert(PF_OUT_F * PF_M / 2 <= PF_LDS, "half the rows in fp32 fit");
@@ -245,42 +245,25 @@ __device__ __forceinline__ u32x4 decode_b(const typename HalfWords<F, HALF>::Buf
     return b;
 }
 
-// A rows of a stage: thread t copies 16-byte chunks (t & 7) and 8 + (t & 7) of rows (t >> 3) and 64 + (t >> 3) (128
-// bytes of a row per 8 lanes). In LDS chunk c = 4 sub + 2 h + q of row r is lane 32 h + r % 32 of operand (sub, q, r /
-// 32); lanes are exchanged by a XOR with 2 (c & 7), which spreads the eight chunks of two rows over the 16 bank groups.
-__device__ __forceinline__ int pf_a_slot(int c, int r)
-{
-    return (((c >> 2) * 2 + (c & 1)) * 4 + (r >> 5)) * 64 + 32 * ((c >> 1) & 1) + ((r & 31) ^ (2 * (c & 7)));
-}
-
+// A rows of a stage: thread t copies 16-byte chunk t & 7 of row t >> 3 of every row block (128 bytes of a row per 8
+// lanes). In LDS chunk c = 4 sub + 2 h + q of row r is lane 32 h + r % 32 of operand (sub, q, r / 32); lanes are exchanged
+// by a XOR with 2 c, which spreads the eight chunks of two rows over the 16 bank groups.
 template <int NMB>
-struct PfStage {
-    static constexpr int NR = NMB > 2 ? 2 : 1;       // row halves (64 rows) that hold rows of the group
-    u32x4 c[NR][2];
-};
-
-template <int NMB>
-__device__ __forceinline__ void pf_stage_load(PfStage<NMB>& st, const uint16_t* rows, const uint32_t (&off)[2], int k0)
+__device__ __forceinline__ void pf_stage_load(u32x4 (&st)[NMB], const uint16_t* rows, int K, uint32_t off, uint32_t last,
+                                              int k0)
 {
-    const char* p = reinterpret_cast<const char*>(rows + k0);
 #pragma unroll
-    for (int j = 0; j < PfStage<NMB>::NR; ++j)
-    {
-        st.c[j][0] = ldg4(p + off[j]);
-        st.c[j][1] = ldg4(p + off[j] + 128);
-    }
+    for (int m = 0; m < NMB; ++m)
+        st[m] = ldg4(reinterpret_cast<const char*>(rows + (size_t)(32 * m) * K + k0) + (m + 1 < NMB ? off : last));
 }
 
 template <int NMB>
-__device__ __forceinline__ void pf_stage_store(const PfStage<NMB>& st, u32x4* __restrict__ lds)
+__device__ __forceinline__ void pf_stage_store(const u32x4 (&st)[NMB], u32x4* __restrict__ lds)
 {
     const int r = threadIdx.x >> 3, c = threadIdx.x & 7;
 #pragma unroll
-    for (int j = 0; j < PfStage<NMB>::NR; ++j)
-    {
-        lds[pf_a_slot(c, r + 64 * j)] = st.c[j][0];
-        lds[pf_a_slot(c + 8, r + 64 * j)] = st.c[j][1];
-    }
+    for (int m = 0; m < NMB; ++m)
+        lds[(((c >> 2) * 2 + (c & 1)) * 4 + m) * 64 + 32 * ((c >> 1) & 1) + (r ^ (2 * c))] = st[m];
 }
 
 // One operand slot of a wave: operand (CI, Q) of the words w is decoded into b while the products of the operand before
@@ -312,13 +295,14 @@ __device__ __forceinline__ void pf_a_read(f16x8 (&a)[NMB], const u32x4* __restri
 #pragma unroll
     for (int m = 0; m < NMB; ++m)
         a[m] = __builtin_bit_cast(f16x8, lds[((2 * j + q) * 4 + m) * 64 + 32 * h +
-                                             ((lane & 31) ^ (2 * (4 * (j & 1) + 2 * h + q)))]);
+                                             ((lane & 31) ^ (2 * (4 * j + 2 * h + q)))]);
     __builtin_amdgcn_sched_barrier(0);        // read a slot ahead of their use
 }
 
-// The unit's k-loop of one wave, NMB 32-row blocks: per stage of 128 k, 4 pairs of tile-rows. The words of a pair are
-// requested four pairs ahead (each register set again right after its use), the A rows one stage ahead; one barrier per
-// stage. WORK false: a wave without columns (past the matrix's last block), which only copies A rows.
+// The unit's k-loop of one wave, NMB 32-row blocks: stages of 64 k, two pairs of tile-rows each, two stages per trip. The
+// words of a pair are requested four pairs ahead (each register set again right after its use), the A rows one stage
+// ahead; one barrier per stage. WORK false: a wave without columns (past the matrix's last block), which only copies A
+// rows.
 template <int F, int HALF, int NMB, bool WORK>
 __device__ __forceinline__ void pf_loop(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc, int cbo,
                                         f32x16 (&acc)[2][NMB])
@@ -330,21 +314,22 @@ __device__ __forceinline__ void pf_loop(const PfJob& jb, const uint8_t* mat_base
     // offsets from wave-uniform addresses; the word before a strip is the tile's last one for its first strip
     const uint32_t strip = (uint32_t)h * row_bytes + (uint32_t)(cbo * 8 + t) * TB + (uint32_t)s * (TB / 4);
     const uint32_t prev = s ? strip - 4 : strip + TB - 4;
-    const int KT = jb.K / PF_KSTEP;
+    const int KT = jb.K / (2 * PF_KSTEP);
     const uint16_t* rows = asrc + (size_t)jb.r0 * jb.K;
-    uint32_t aoff[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-        aoff[j] = 2u * ((uint32_t)min((int)(threadIdx.x >> 3) + 64 * j, jb.nr - 1) * (uint32_t)jb.K + 8u * (threadIdx.x & 7));
-    PfStage<NMB> st;
-    typename S::Buf w[PF_SUBS];
+    // the thread's row in a row block; in the last block rows past the group's end read its last row
+    const int r = threadIdx.x >> 3;
+    const uint32_t off = 2u * ((uint32_t)r * (uint32_t)jb.K + 8u * (threadIdx.x & 7));
+    const uint32_t last = 2u * ((uint32_t)min(r, jb.nr - 1 - 32 * (NMB - 1)) * (uint32_t)jb.K + 8u * (threadIdx.x & 7));
+    u32x4 st[NMB];
+    typename S::Buf w[2 * PF_SUBS];
     u32x4 b0, b1;
     f16x8 a0[NMB], a1[NMB];
-    pf_stage_load<NMB>(st, rows, aoff, 0);
+    pf_stage_load<NMB>(st, rows, jb.K, off, last, 0);
     if (WORK)
     {
 #pragma unroll
-        for (int j = 0; j < PF_SUBS; ++j) load_half<F, HALF>(w[j], mat_base + (size_t)(2 * j) * row_bytes, strip, prev);
+        for (int j = 0; j < 2 * PF_SUBS; ++j)
+            load_half<F, HALF>(w[j], mat_base + (size_t)(2 * j) * row_bytes, strip, prev);
         // the pipeline starts with an operand of zeros (its products add nothing)
         b1 = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
@@ -354,30 +339,35 @@ __device__ __forceinline__ void pf_loop(const PfJob& jb, const uint8_t* mat_base
     step_barrier();
     for (int i = 0; i < KT; ++i)
     {
-        const int in = min(i + 1, KT - 1);          // past the last stage: its own loads again, never used
-        const u32x4* lds = pf_lds + (i & 1) * PF_ST_U4;
-        pf_stage_load<NMB>(st, rows, aoff, in * PF_KSTEP);
-        if (WORK)
+        const int in = min(i + 1, KT - 1);          // past the last trip: its own loads again, never used
+        const uint8_t* pn = mat_base + (size_t)(4 * PF_SUBS) * in * row_bytes;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
         {
-            const uint8_t* pn = mat_base + (size_t)(2 * PF_SUBS) * in * row_bytes;
-#pragma unroll
-            for (int j = 0; j < PF_SUBS; ++j)
+            const u32x4* lds = pf_lds + g * PF_ST_U4;
+            pf_stage_load<NMB>(st, rows, jb.K, off, last, g == 0 ? (2 * i + 1) * PF_KSTEP : 2 * in * PF_KSTEP);
+            if (WORK)
             {
-                // the words stay allocated until here (a load in flight into a register that is free again would force
-                // a wait)
 #pragma unroll
-                for (int k = 0; k < S::NW; ++k) asm volatile("" :: "v"(w[j][k]));
-                pf_a_read<NMB>(a0, lds, j, 0);
-                pf_slot<F, HALF, 0, 0, NMB>(w[j], b0, b1, a1, acc);
-                pf_slot<F, HALF, 1, 0, NMB>(w[j], b1, b0, a0, acc);
-                pf_a_read<NMB>(a1, lds, j, 1);
-                pf_slot<F, HALF, 0, 1, NMB>(w[j], b0, b1, a0, acc);
-                pf_slot<F, HALF, 1, 1, NMB>(w[j], b1, b0, a1, acc);
-                load_half<F, HALF>(w[j], pn + (size_t)(2 * j) * row_bytes, strip, prev);
+                for (int j = 0; j < PF_SUBS; ++j)
+                {
+                    typename S::Buf& wj = w[PF_SUBS * g + j];
+                    // the words stay allocated until here (a load in flight into a register that is free again would
+                    // force a wait)
+#pragma unroll
+                    for (int k = 0; k < S::NW; ++k) asm volatile("" :: "v"(wj[k]));
+                    pf_a_read<NMB>(a0, lds, j, 0);
+                    pf_slot<F, HALF, 0, 0, NMB>(wj, b0, b1, a1, acc);
+                    pf_slot<F, HALF, 1, 0, NMB>(wj, b1, b0, a0, acc);
+                    pf_a_read<NMB>(a1, lds, j, 1);
+                    pf_slot<F, HALF, 0, 1, NMB>(wj, b0, b1, a0, acc);
+                    pf_slot<F, HALF, 1, 1, NMB>(wj, b1, b0, a1, acc);
+                    load_half<F, HALF>(wj, pn + (size_t)(2 * (PF_SUBS * g + j)) * row_bytes, strip, prev);
+                }
             }
+            pf_stage_store<NMB>(st, pf_lds + (1 - g) * PF_ST_U4);
+            step_barrier();
         }
-        pf_stage_store<NMB>(st, pf_lds + ((i + 1) & 1) * PF_ST_U4);
-        step_barrier();
     }
     if (WORK)
 #pragma unroll
@@ -415,11 +405,11 @@ __device__ __forceinline__ void pf_out(const GvArgs& a, const PfJob& jb, const f
                 }
         step_barrier();
         // 16-byte pieces: PPR per row; piece q of a row is in 128-column block q / PPB
-        constexpr int PPR = PF_COLS * ES / 16, PPB = PPR / 4;
+        constexpr int PPR = PF_COLS * ES / 16, PPB = PPR / 2;
         const int rows = min(jb.nr - 32 * m0, 32 * RB);
         for (int i = threadIdx.x; i < rows * PPR; i += PF_WAVES * 64)
         {
-            const int row = i / PPR, q = i % PPR, cbo = 4 * jb.cb + q / PPB;
+            const int row = i / PPR, q = i % PPR, cbo = 2 * jb.cb + q / PPB;
             if (cbo >= jb.nb128) continue;
             const u32x4 v = *reinterpret_cast<const u32x4*>(lds + row * RS + q * 16);
             const size_t r = (size_t)(jb.r0 + 32 * m0 + row);
@@ -461,7 +451,7 @@ template <bool DOWN, int F>
 __device__ __forceinline__ void pf_unit_half(const GvArgs& a, const PfJob& jb, const uint8_t* base, const uint16_t* asrc,
                                              int wave)
 {
-    const int cbo = 4 * jb.cb + (wave >> 1);
+    const int cbo = 2 * jb.cb + (wave >> 1);
     if (wave & 1) pf_unit_rows<DOWN, F, 1>(a, jb, base, asrc, cbo);
     else pf_unit_rows<DOWN, F, 0>(a, jb, base, asrc, cbo);
 }
@@ -470,12 +460,12 @@ template <bool DOWN>
 __global__ __launch_bounds__(PF_WAVES * 64, 2) void k_pf_gemm(GvArgs a)
 {
     const int nb128 = DOWN ? a.NBH : a.NB;     // 128-column blocks of the output
-    const int NB4 = (nb128 + 3) / 4;
+    const int NB2 = (nb128 + 1) / 2;
     const int lid = xcd_block(blockIdx.x, gridDim.x);
     PfJob jb;
     jb.nb128 = nb128;
-    if (DOWN) { jb.g = lid / NB4; jb.mat = 2; jb.cb = lid % NB4; }
-    else { jb.g = lid / (2 * NB4); jb.mat = (lid / NB4) & 1; jb.cb = lid % NB4; }
+    if (DOWN) { jb.g = lid / NB2; jb.mat = 2; jb.cb = lid % NB2; }
+    else { jb.g = lid / (2 * NB2); jb.mat = (lid / NB2) & 1; jb.cb = lid % NB2; }
     if (jb.g >= *a.ngroups) return;
     jb.e = a.groups[3 * jb.g];
     if (group_skipped(a, jb.e)) return;
@@ -898,7 +888,7 @@ int launch_prefill_experts(const MoeShape& m, const void* x, const bmx_routes* r
         if (!(stages & (1 << st))) continue;
         GvArgs b = a;
         b.filter = f;
-        hipLaunchKernelGGL(k_pf_gemm<false>, dim3((unsigned)(p.G_max * 2 * ((p.NB + 3) / 4))), dim3(PF_WAVES * 64), 0, s, b);
+        hipLaunchKernelGGL(k_pf_gemm<false>, dim3((unsigned)(p.G_max * 2 * ((p.NB + 1) / 2))), dim3(PF_WAVES * 64), 0, s, b);
     }
     if (stages & (1 << BMX_STAGE_ACT)) rc = launch_epilogue(a, BMX_STAGE_ACT, s);
     for (int f = 0; f < 3 && !rc; ++f)
@@ -907,7 +897,7 @@ int launch_prefill_experts(const MoeShape& m, const void* x, const bmx_routes* r
         if (!(stages & (1 << st))) continue;
         GvArgs b = a;
         b.filter = f;
-        hipLaunchKernelGGL(k_pf_gemm<true>, dim3((unsigned)(p.G_max * ((p.NBH + 3) / 4))), dim3(PF_WAVES * 64), 0, s, b);
+        hipLaunchKernelGGL(k_pf_gemm<true>, dim3((unsigned)(p.G_max * ((p.NBH + 1) / 2))), dim3(PF_WAVES * 64), 0, s, b);
     }
     if (!rc && (stages & (1 << BMX_STAGE_COMBINE))) rc = launch_epilogue(a, BMX_STAGE_COMBINE, s);
     if (!rc && (stages & (1 << BMX_STAGE_DOWN_OUT))) rc = launch_epilogue(a, BMX_STAGE_DOWN_OUT, s);
