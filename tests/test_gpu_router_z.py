@@ -53,6 +53,26 @@ def test_router_logits_projection(cuda, oracle, T, E, H):
     assert frac < 0.01
 
 
+@pytest.mark.parametrize("T,E,H", [(1024, 384, 576),     # 96 tiles of 64 x 64, H = 64 mod 128
+                                   (1025, 383, 2112),    # the same tiles, one row and one expert past them
+                                   (1023, 321, 64),      # one step per quarter
+                                   (511, 256, 1088),     # 128 tiles of 32 x 32
+                                   (480, 256, 192),      # just below: 16 experts a tile
+                                   (9, 250, 5184)])      # one row past the kernel of few rows, H past its first trip
+def test_router_logits_same_in_every_tile(cuda, oracle, T, E, H):
+    """A token's logits are the same bits whatever tile its call takes: the call against calls of 31, 8 and 3 tokens."""
+    import bmx
+    z = torch.randn((T, H), device=cuda).half()
+    W = (torch.randn((E, H), device=cuda) / H ** 0.5).half()
+    say("router logits tiles", T, E, H)
+    got = bmx.ops.router_logits(z, W)
+    for n in (31, 8, 3):
+        few = torch.cat([bmx.ops.router_logits(z[t:t + n], W) for t in range(0, T, n)])
+        assert torch.equal(got.view(torch.int16), few.view(torch.int16))
+    rows = np.r_[0:T:37, T - 1]
+    check_logits(got.cpu().numpy()[rows], z.cpu().numpy()[rows], W.cpu().numpy(), oracle)
+
+
 def test_router_logits_prefill_rows(cuda, oracle):
     """The 8192-token DeepSeek-shaped chunk: every row projected (E 384, H 4096), a sample of rows checked."""
     import bmx
