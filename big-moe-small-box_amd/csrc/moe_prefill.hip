@@ -112,16 +112,6 @@ static dim3 prep_tok_grid(int T, int H)
     return dim3((unsigned)std::max(1L, (units + 15) / 16));
 }
 
-// ---- B fragments in LDS (mid-size path) -----------------------------------------------------------------------------
-// B stage: fragment f = tile-row * 8 + 32-column block of the 256, 64 lanes x 16 B; lane L's 16 B at slot f * 64 +
-//          bsw(f, L), bsw(f, L) = L ^ ((L >> 4) & 1) ^ ((f & 1) << 3): a bijection on each 16-lane block (the MFMA reads
-//          stay conflict-free) that spreads the 16 lanes of a decode store over 16 bank groups.
-constexpr int PF_B_U4 = 4 * 8 * 64;
-__shared__ u32x4 pf_b0[PF_B_U4];
-__shared__ u32x4 pf_b1[PF_B_U4];
-
-__device__ __forceinline__ int bsw(int f, int L) { return L ^ ((L >> 4) & 1) ^ ((f & 1) << 3); }
-
 // Step barrier: the wave's LDS operations are done (its global loads, register prefetches for later steps, may still be in
 // flight; the compiler waits for those where their registers are used).
 __device__ __forceinline__ void step_barrier()
@@ -130,50 +120,6 @@ __device__ __forceinline__ void step_barrier()
     __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0); vmcnt (63) and expcnt (7) at their maxima: no wait
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-}
-
-// ---- B operand: half a strip decoded into fragments -------------------------------------------------------------------
-// Fragment (tile-row kt, 32-column block nb) holds, for MFMA lane L, the 8 input rows 8 (L / 32) .. + 7 of column
-// 32 nb + L % 32 as 4 dwords (rows 2d, 2d + 1 in dword d). Stream positions 32 HALF .. 32 HALF + 31 of a lane's strip are
-// columns HALF and HALF + 2 of its four, all 16 rows: two columns' worth of fragments. col0: the first column of the
-// lane's 128-column half of the block.
-// The lane index as a value the compiler cannot hoist: LDS addresses derived from it are recomputed where they are used
-// (a few VALU per step) instead of being kept live across the k-loop, which costs the mid-size kernel its occupancy.
-__device__ __forceinline__ int fresh_lane()
-{
-    int l = threadIdx.x & 63;
-    asm volatile("" : "+v"(l));
-    return l;
-}
-
-template <int F, int HALF>
-__device__ __forceinline__ void decode_half(const uint32_t (&own)[Fmt<F>::TB / 16], u32x4* __restrict__ stage, int kt,
-                                            int col0, int lane)
-{
-    constexpr int NW = Fmt<F>::TB / 16;
-    // every word of the window is consumed here (a half strip reads only some of them): keeps the prefetched registers
-    // allocated until now instead of reused while their load is in flight, which would force a wait on it
-#pragma unroll
-    for (int k = 0; k < NW; ++k) asm volatile("" :: "v"(own[k]));
-    const uint32_t prev = __builtin_amdgcn_mov_dpp(own[NW - 1], 0x93, 0xf, 0xf, false);
-    uint32_t fr[2][8];
-#pragma unroll
-    for (int j8 = 32 * HALF; j8 < 32 * HALF + 32; j8 += 8)
-    {
-        uint32_t w[4];
-        oct_weights<F>(prev, own, j8, w);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) fr[strip_cidx(j8 + 2 * q) >> 1][strip_dw(j8 + 2 * q)] = w[q];
-    }
-#pragma unroll
-    for (int ci = 0; ci < 2; ++ci)
-    {
-        const int col = col0 + lane_col(lane, HALF + 2 * ci);
-        const int f = kt * 8 + (col >> 5);
-        u32x4* fp = stage + f * 64;
-        fp[bsw(f, col & 31)] = u32x4{fr[ci][0], fr[ci][1], fr[ci][2], fr[ci][3]};
-        fp[bsw(f, (col & 31) + 32)] = u32x4{fr[ci][4], fr[ci][5], fr[ci][6], fr[ci][7]};
-    }
 }
 
 // ---- grouped GEMM ----------------------------------------------------------------------------------------------------
@@ -486,124 +432,97 @@ __global__ __launch_bounds__(PF_WAVES * 64, 2) void k_pf_gemm(GvArgs a)
     }
 }
 
-// ---- mid-size grouped GEMM: groups of <= 32 rows, every wave decodes and multiplies ------------------------------------
-// For decode batches of several tokens (a few rows per expert): work unit = (group of <= 32 rows, matrix, 256-column block,
-// k-split). 8 waves; per k-step of 64 each wave decodes half a strip per tile-row exactly as a prefill decode wave does
-// (same B fragment layout, pf_b0 / pf_b1), copies 8 bytes of the A rows, and, from the previous step's stage, runs the 4
-// MFMAs (32 rows x 32 columns, k 16 each) of its 32-column block. One barrier per step; the fp32 products of each k-split
-// go to the partial layout the epilogues sum in split order.
+// ---- mid-size grouped GEMM: groups of <= 32 rows, every wave on its own ------------------------------------------------
+// For decode batches of several tokens (a few rows per expert): a wave's unit is (group of <= 32 rows, matrix, 128-column
+// block, k-split). Per pair of tile-rows (32 k) a lane holds one whole strip, four columns of 16 rows, and decodes it
+// straight into the B operands of eight v_mfma_f32_32x32x16_f16 (lane L: tile-row L / 32, as in the prefill GEMM); the A
+// operands, 32 bytes of a row per lane, come from memory (the L1 and L2 hold the few rows). Nothing goes through LDS and
+// no wave waits for another, so three waves per SIMD keep the VALU busy, which bounds it: 230 VALU per strip of 64 weights
+// and lane. The fp32 products of each k-split go to the partial layout the epilogues sum in split order. The workgroup's
+// four waves take consecutive column blocks of the same rows. Against eight waves that decoded
+// into LDS between barriers (and spilled): 77 tokens 679 -> 591 us, 8 tokens 195 -> 165, 16 tokens on ~12 experts 102 -> 86.
 constexpr int MID_M = 32;
-constexpr int MID_WAVES = 8;
-constexpr int MID_A_U4 = MID_M * 8;
-__shared__ u32x4 mid_a0[MID_A_U4];
-__shared__ u32x4 mid_a1[MID_A_U4];
-__device__ __forceinline__ u32x4* mid_a_stage(int s) { return s == 0 ? mid_a0 : mid_a1; }
+constexpr int MID_WAVES = 4;
+constexpr int MID_D = 2;                      // strips of trellis words in flight per wave
 
-struct MidArow {
-    uint32_t d[2];
-};
-
-// lane's 8 bytes of the A rows of a step: row 4 wave + lane / 16, bytes 8 (lane % 16) of the row's 128 (64 inputs)
-__device__ __forceinline__ void mid_a_fetch(MidArow& r, const uint16_t* rowp, int k0)
+// B operand (C, Q) of a whole strip: the eight input rows 8 Q .. + 7 of strip column C
+template <int F, int C, int Q>
+__device__ __forceinline__ u32x4 strip_b(uint32_t prev, const uint32_t (&own)[Fmt<F>::TB / 16])
 {
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(rowp + k0);
-    r.d[0] = ldg(p, 0);
-    r.d[1] = ldg(p, 1);
-}
-
-__device__ __forceinline__ void mid_a_store(const MidArow& r, u32x4* __restrict__ stage, int lane)
-{
-    const int row = 4 * (threadIdx.x >> 6) + (lane >> 4), piece = lane & 15;
-    uint2* p = reinterpret_cast<uint2*>(stage + row * 8 + ((piece >> 1) ^ ((row >> 1) & 7))) + (piece & 1);
-    *p = make_uint2(r.d[0], r.d[1]);
-}
-
-// the wave's 32-column block of one step: 4 MFMAs, k 16 each, into one accumulator (the MFMA units are lightly used
-// here; a second accumulator would cost the 16 VGPRs that keep the kernel at 128)
-__device__ __forceinline__ void mid_mfma_step(const u32x4* __restrict__ sa, const u32x4* __restrict__ sb, f32x16& acc,
-                                              int lane)
-{
-    const int wave = threadIdx.x >> 6;
-    f16x8 fa[4], fb[4];
+    constexpr RingTab<F> tab;
+    u32x4 b;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int g = 0; g < 4; ++g)
     {
-        const int slot = (2 * ks + (lane >> 5)) ^ ((lane >> 1) & 7), fi = ks * 8 + wave;
-        fa[ks] = __builtin_bit_cast(f16x8, sa[(lane & 31) * 8 + slot]);
-        fb[ks] = __builtin_bit_cast(f16x8, sb[fi * 64 + bsw(fi, lane)]);
+        const int j = 32 * (C & 1) + 8 * g + 4 * (C >> 1) + 2 * Q;      // strip_cidx(j) = C, strip_dw(j) = g + 4 Q
+        b[g] = cb_pair(win_state(prev, own, tab.q[j]), win_state(prev, own, tab.q[j + 1]));
     }
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[ks], fb[ks], acc, 0, 0, 0);
+    return b;
 }
 
-// steps s0 .. s0 + n - 1 of the unit; straight-line like pf_decoder (loads past the last step re-read it)
-template <int F, int HALF>
-__device__ __forceinline__ void mid_run(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc, int s0, int n,
-                                        f32x16& acc)
+template <int F, int C, int Q>
+__device__ __forceinline__ void mid_mul(uint32_t prev, const uint32_t (&own)[Fmt<F>::TB / 16], const u32x4& a, f32x16 (&acc)[4])
+{
+    acc[C] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, strip_b<F, C, Q>(prev, own)),
+                                                    acc[C], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);        // one operand's decode at a time: the registers of two would cost a wave per SIMD
+}
+
+// pairs of tile-rows s0 .. s0 + n - 1 of the wave's unit (n > 0). ap: the lane's A row at k 16 (L / 32)
+template <int F>
+__device__ __forceinline__ void mid_run(const PfJob& jb, const uint8_t* mat_base, const uint16_t* ap, int s0, int n,
+                                        f32x16 (&acc)[4])
 {
     constexpr int TB = Fmt<F>::TB, NW = TB / 16;
-    const int lane = threadIdx.x & 63, d = threadIdx.x >> 6;
-    const int h = lane >> 5, t = (lane >> 2) & 7, sl = lane & 3;
-    const int kt = 2 * (d >> 2) + h, th = (d >> 1) & 1;
-    const int tcol = min(2 * jb.cb + th, jb.nb128 - 1);
-    const size_t row_bytes = (size_t)(jb.N / 16) * TB, step_bytes = 4 * row_bytes;
-    const uint8_t* p = mat_base + (size_t)kt * row_bytes + (size_t)(tcol * 8 + t) * TB + sl * (TB / 4);
-    const int arow = 4 * d + (lane >> 4);
-    const uint16_t* rowp = asrc + (size_t)(jb.r0 + min(arow, jb.nr - 1)) * jb.K + 4 * (lane & 15);
-    auto wp = [&](int i) { return p + (size_t)(s0 + min(i, n - 1)) * step_bytes; };
-    auto ak = [&](int i) { return 64 * (s0 + min(i, n - 1)); };
-    // the lane index once per call, opaque to the compiler: the LDS addresses derived from it are this copy's own (the
-    // compiler cannot merge them above the format switch, where every copy's set would be live at once)
-    const int ln = fresh_lane();
-    uint32_t w0[NW], w1[NW];
-    MidArow a0, a1;
-    mid_a_fetch(a0, rowp, ak(0));
-    mid_a_fetch(a1, rowp, ak(1));
-    load_words(w0, wp(0));
-    load_words(w1, wp(1));
-    decode_half<F, HALF>(w0, pf_b0, kt, 128 * th, ln);
-    mid_a_store(a0, mid_a0, ln);
-    step_barrier();
-    // step i: the MFMAs of stage i % 2, the decode of step i + 1 into the other stage, the fetch of step i + 2 (two
-    // register sets: the kernel fits 128 VGPRs, so two workgroups share a CU)
-    for (int i = 0; i < n; i += 2)
-    {
-        mid_a_fetch(a0, rowp, ak(i + 2));
-        load_words(w0, wp(i + 2));
-        mid_mfma_step(mid_a0, pf_b0, acc, ln);
-        decode_half<F, HALF>(w1, pf_b1, kt, 128 * th, ln);
-        mid_a_store(a1, mid_a1, ln);
-        step_barrier();
-        if (i + 1 >= n) break;
-        mid_a_fetch(a1, rowp, ak(i + 3));
-        load_words(w1, wp(i + 3));
-        mid_mfma_step(mid_a1, pf_b1, acc, ln);
-        decode_half<F, HALF>(w0, pf_b0, kt, 128 * th, ln);
-        mid_a_store(a0, mid_a0, ln);
-        step_barrier();
-    }
+    const int lane = threadIdx.x & 63, h = lane >> 5, t = (lane >> 2) & 7, s = lane & 3;
+    const size_t pair_bytes = (size_t)(jb.N / 16) * TB * 2;
+    const uint8_t* p = mat_base + (size_t)s0 * pair_bytes + h * (pair_bytes / 2) + (size_t)(jb.cb * 8 + t) * TB + s * (TB / 4);
+    ap += 32 * s0;
+    uint32_t w[MID_D][NW];
+    u32x4 a[MID_D][2];
+    // past the last pair: the last one again
+    auto fetch = [&](int d, int i) {
+        const int j = min(i, n - 1);
+        load_words(w[d], p + (size_t)j * pair_bytes);
+        a[d][0] = ldg4(ap + 32 * j);
+        a[d][1] = ldg4(ap + 32 * j + 8);
+    };
+#pragma unroll
+    for (int d = 0; d < MID_D; ++d) fetch(d, d);
+    for (int i = 0; i < n; i += MID_D)
+#pragma unroll
+        for (int d = 0; d < MID_D; ++d)
+        {
+            if (i + d >= n) break;
+            const uint32_t prev = __builtin_amdgcn_mov_dpp(w[d][NW - 1], 0x93, 0xf, 0xf, false);
+            mid_mul<F, 0, 0>(prev, w[d], a[d][0], acc);
+            mid_mul<F, 1, 0>(prev, w[d], a[d][0], acc);
+            mid_mul<F, 2, 0>(prev, w[d], a[d][0], acc);
+            mid_mul<F, 3, 0>(prev, w[d], a[d][0], acc);
+            mid_mul<F, 0, 1>(prev, w[d], a[d][1], acc);
+            mid_mul<F, 1, 1>(prev, w[d], a[d][1], acc);
+            mid_mul<F, 2, 1>(prev, w[d], a[d][1], acc);
+            mid_mul<F, 3, 1>(prev, w[d], a[d][1], acc);
+            fetch(d, i + d + MID_D);
+        }
 }
 
-template <int F>
-__device__ __forceinline__ void mid_run_any(const PfJob& jb, const uint8_t* mat_base, const uint16_t* asrc, int s0, int n,
-                                            f32x16& acc)
-{
-    if ((threadIdx.x >> 6) & 1) mid_run<F, 1>(jb, mat_base, asrc, s0, n, acc);
-    else mid_run<F, 0>(jb, mat_base, asrc, s0, n, acc);
-}
-
-// One unit of the mid-size GEMM: (group or heavy-expert chunk, matrix, 256-column block, k-split) from its index lid.
+// One unit of the mid-size GEMM: (group or heavy-expert chunk, matrix, four 128-column blocks, k-split) from its index lid.
 template <bool DOWN>
 __device__ __forceinline__ void mid_unit(const GvArgs& a, int lid)
 {
     const int nb128 = DOWN ? a.NBH : a.NB;
-    const int NB2 = (nb128 + 1) / 2, KS = DOWN ? a.KS_dn : a.KS_gu;
+    const int NB4 = (nb128 + MID_WAVES - 1) / MID_WAVES, KS = DOWN ? a.KS_dn : a.KS_gu;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int ksp = lid % KS;
     lid /= KS;
     PfJob jb;
     jb.nb128 = nb128;
-    if (DOWN) { jb.g = lid / NB2; jb.mat = 2; jb.cb = lid % NB2; }
-    else { jb.g = lid / (2 * NB2); jb.mat = (lid / NB2) & 1; jb.cb = lid % NB2; }
+    jb.cb = lid % NB4 * MID_WAVES + wave;
+    lid /= NB4;
+    jb.mat = DOWN ? 2 : lid & 1;
+    jb.g = DOWN ? lid : lid >> 1;
+    if (jb.cb >= nb128) return;
     if (a.split_min)
     {
         // split path: units over (unique expert, chunk of 32 rows); only the heavy experts' rows are computed here
@@ -627,41 +546,39 @@ __device__ __forceinline__ void mid_unit(const GvArgs& a, int lid)
     jb.ex = jb.e == a.E ? a.shared : a.experts + jb.e;
     jb.K = DOWN ? a.I : a.H;
     jb.N = DOWN ? a.H : a.I;
-    const int n = jb.K / 64 / KS, s0 = ksp * n;
+    const int lane = threadIdx.x & 63, n = jb.K / 32 / KS, s0 = ksp * n;
     const uint16_t* asrc = DOWN ? a.act_rows : a.xt + (size_t)jb.mat * a.R_max * a.H;
+    const uint16_t* ap = asrc + (size_t)(jb.r0 + min(lane & 31, jb.nr - 1)) * jb.K + 16 * (lane >> 5);
     const uint8_t* base = reinterpret_cast<const uint8_t*>(jb.ex->tr[jb.mat]);
-    f32x16 acc = f32x16{};
+    f32x16 acc[4] = {};
     switch (jb.ex->fmt[jb.mat])
     {
-        case BMX_TF_K2: mid_run_any<BMX_TF_K2>(jb, base, asrc, s0, n, acc); break;
-        case BMX_TF_K25: mid_run_any<BMX_TF_K25>(jb, base, asrc, s0, n, acc); break;
-        case BMX_TF_K3: mid_run_any<BMX_TF_K3>(jb, base, asrc, s0, n, acc); break;
-        default: mid_run_any<BMX_TF_K4>(jb, base, asrc, s0, n, acc); break;
+        case BMX_TF_K2: mid_run<BMX_TF_K2>(jb, base, ap, s0, n, acc); break;
+        case BMX_TF_K25: mid_run<BMX_TF_K25>(jb, base, ap, s0, n, acc); break;
+        case BMX_TF_K3: mid_run<BMX_TF_K3>(jb, base, ap, s0, n, acc); break;
+        default: mid_run<BMX_TF_K4>(jb, base, ap, s0, n, acc); break;
     }
-    // accumulator element v of lane L: row 8 (v / 4) + 4 (L / 32) + v % 4, column L % 32 of the wave's 32-column block
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int cbo = 2 * jb.cb + (wave >> 2);
-    if (cbo >= nb128) return;
-    const int col = 32 * (wave & 3) + (lane & 31);
-    // row stride of the partial layout (floats); the lane's first row 4 (lane / 32)
+    // accumulator element v of lane L: row 8 (v / 4) + 4 (L / 32) + v % 4, column lane_col(L, c); row stride of the partial
+    // layout in floats
     const int rs = DOWN ? a.NBH * 128 : a.NB * 256;
     const size_t r0 = (size_t)ksp * a.R_max + jb.r0 + 4 * (lane >> 5);
-    float* out = (DOWN ? a.part_dn + cbo * 128 : a.part_gu + cbo * 256 + jb.mat * 128) + r0 * rs + col;
+    float* out = (DOWN ? a.part_dn + jb.cb * 128 : a.part_gu + jb.cb * 256 + jb.mat * 128) + r0 * rs + lane_col(lane, 0);
 #pragma unroll
     for (int v = 0; v < 16; ++v)
     {
         const int dr = 8 * (v >> 2) + (v & 3);
         if (dr + 4 * (lane >> 5) >= jb.nr) continue;
-        out[(size_t)dr * rs] = acc[v];
+        *reinterpret_cast<float2*>(out + (size_t)dr * rs) = make_float2(acc[0][v], acc[1][v]);
+        *reinterpret_cast<float2*>(out + (size_t)dr * rs + 8) = make_float2(acc[2][v], acc[3][v]);
     }
 }
 
 template <bool DOWN>
-__global__ __launch_bounds__(MID_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_mid_gemm(GvArgs a)
+__global__ __launch_bounds__(MID_WAVES * 64, 3) void k_mid_gemm(GvArgs a)
 {
     if (!a.split_min)
     {
-        mid_unit<DOWN>(a, xcd_block(blockIdx.x, gridDim.x));
+        mid_unit<DOWN>(a, blockIdx.x);
         return;
     }
     // split path: a grid of at most MID_SPLIT_WGS workgroups loops over the units of the call's unique experts, so a call
@@ -669,13 +586,9 @@ __global__ __launch_bounds__(MID_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
     // reach split_min rows)
     if (a.split_min > a.T + 1 && 2 * a.offsets[a.NE] < a.split_ratio2 * *a.nuniq) return;
     const int nb128 = DOWN ? a.NBH : a.NB;
-    const int per = (DOWN ? 1 : 2) * ((nb128 + 1) / 2) * (DOWN ? a.KS_dn : a.KS_gu);
+    const int per = (DOWN ? 1 : 2) * ((nb128 + MID_WAVES - 1) / MID_WAVES) * (DOWN ? a.KS_dn : a.KS_gu);
     const int units = *a.nuniq * a.split_chunks * per;
-    for (int lid = blockIdx.x; lid < units; lid += gridDim.x)
-    {
-        mid_unit<DOWN>(a, lid);
-        __syncthreads();          // the unit's LDS stages are read out before the next unit writes them
-    }
+    for (int lid = blockIdx.x; lid < units; lid += gridDim.x) mid_unit<DOWN>(a, lid);
 }
 
 // ---- plan and launch -------------------------------------------------------------------------------------------------
@@ -713,15 +626,17 @@ struct MidPlan {
     size_t xt_bytes, part_gu_bytes, act_bytes, part_dn_bytes;
 };
 
-// k-split: the most splits that keep at least 16 k-steps each, gate / up (BMX_MID_MIN_STEPS) and down
-// (BMX_MID_MIN_STEPS_DN) (the routing, unknown here, may put all rows on a few experts; splits keep the workgroup count
-// up then, at the price of partial sums the epilogue adds). Measured (layer us; 8 / 16 / 32 steps for down): 16 tokens
-// on ~10 experts of H 4096, I 2048: 103.7 / 104.4 / 106.6; GLM-shaped 8 tokens: 218 / 214 / 214; DeepSeek-shaped 16
-// tokens: 298 / 292 / 295. Gate / up at 8 or 32 steps: 5-7 % slower than 16 on the first.
-static int mid_split(int ksteps, bool down)
+// k-split: the most splits that keep at least min_steps k-steps of 64 each, gate / up (BMX_MID_MIN_STEPS) and down
+// (BMX_MID_MIN_STEPS_DN). Splits even out the SIMDs' shares (the routing, unknown here, may put all rows on a few experts),
+// at the price of partial sums that the epilogues add. Up to MID_FEW_ROWS dispatch rows the partials are small: 8 and 4
+// steps, above them 16 and 8. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60 experts of H 4096,
+// I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I 2048) 8 x 4: 86, 4 x 4:
+// 92, 16 x 4: 95, 16 x 16: 103; 77 tokens (693 rows, 255 experts) 16 x 8: 591, 8 x 8: 608, 16 x 4: 609, 32 x 8: 600.
+constexpr int MID_FEW_ROWS = 160;
+static int mid_split(int ksteps, bool down, int rows)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
-    const int min_steps = (v && *v) ? atoi(v) : 16;
+    const int min_steps = (v && *v) ? atoi(v) : (rows <= MID_FEW_ROWS ? 8 : 16) / (down ? 2 : 1);
     for (int d = ksteps; d > 1; --d)
         if (ksteps % d == 0 && ksteps / d >= min_steps) return d;
     return 1;
@@ -734,8 +649,8 @@ static MidPlan mid_plan(const MoeShape& m)
     p.NBH = m.H / 128;
     p.G_max = groups_max(m.T, m.topk, m.E, m.shared, MID_M);
     p.R_max = m.T * m.topk + (m.shared ? m.T : 0);
-    p.KS_gu = mid_split(m.H / 64, false);
-    p.KS_dn = mid_split(m.I / 64, true);
+    p.KS_gu = mid_split(m.H / 64, false, p.R_max);
+    p.KS_dn = mid_split(m.I / 64, true, p.R_max);
     p.xt_bytes = (size_t)2 * p.R_max * m.H * 2;
     p.part_gu_bytes = (size_t)p.KS_gu * p.R_max * p.NB * 256 * 4;
     p.act_bytes = (size_t)p.R_max * m.I * 2;
@@ -744,6 +659,9 @@ static MidPlan mid_plan(const MoeShape& m)
 }
 
 int mid_rows_per_group() { return MID_M; }
+
+// workgroups across a matrix's 128-column blocks
+static int mid_blocks(int nb128) { return (nb128 + MID_WAVES - 1) / MID_WAVES; }
 
 size_t mid_ws_bytes(const MoeShape& m)
 {
@@ -793,7 +711,7 @@ int launch_mid_experts(const MoeShape& m, const void* x, const bmx_routes* r, fl
         if (!(stages & (1 << st))) continue;
         GvArgs b = a;
         b.filter = f;
-        hipLaunchKernelGGL(k_mid_gemm<false>, dim3((unsigned)(p.G_max * 2 * ((p.NB + 1) / 2) * p.KS_gu)),
+        hipLaunchKernelGGL(k_mid_gemm<false>, dim3((unsigned)(p.G_max * 2 * mid_blocks(p.NB) * p.KS_gu)),
                            dim3(MID_WAVES * 64), 0, s, b);
     }
     if (stages & (1 << BMX_STAGE_ACT)) rc = launch_epilogue(a, BMX_STAGE_ACT, s);
@@ -803,7 +721,7 @@ int launch_mid_experts(const MoeShape& m, const void* x, const bmx_routes* r, fl
         if (!(stages & (1 << st))) continue;
         GvArgs b = a;
         b.filter = f;
-        hipLaunchKernelGGL(k_mid_gemm<true>, dim3((unsigned)(p.G_max * ((p.NBH + 1) / 2) * p.KS_dn)),
+        hipLaunchKernelGGL(k_mid_gemm<true>, dim3((unsigned)(p.G_max * mid_blocks(p.NBH) * p.KS_dn)),
                            dim3(MID_WAVES * 64), 0, s, b);
     }
     if (!rc && (stages & (1 << BMX_STAGE_COMBINE))) rc = launch_epilogue(a, BMX_STAGE_COMBINE, s);
@@ -830,11 +748,11 @@ void launch_split_mid(const GvArgs& a, int stage, int nu_max, hipStream_t s)
     if (stage == BMX_STAGE_PREP)
         hipLaunchKernelGGL(k_pf_prep, prep_grid(a.R_max, a.H), dim3(256), 0, s, a);
     else if (stage == BMX_STAGE_DOWN || stage == BMX_STAGE_DOWN_RESIDENT || stage == BMX_STAGE_DOWN_STAGED)
-        hipLaunchKernelGGL(k_mid_gemm<true>, dim3((unsigned)std::min(MID_SPLIT_WGS, units * ((a.NBH + 1) / 2) * a.KS_dn)),
+        hipLaunchKernelGGL(k_mid_gemm<true>, dim3((unsigned)std::min(MID_SPLIT_WGS, units * mid_blocks(a.NBH) * a.KS_dn)),
                            dim3(MID_WAVES * 64), 0, s, a);
     else
         hipLaunchKernelGGL(k_mid_gemm<false>,
-                           dim3((unsigned)std::min(MID_SPLIT_WGS, units * 2 * ((a.NB + 1) / 2) * a.KS_gu)),
+                           dim3((unsigned)std::min(MID_SPLIT_WGS, units * 2 * mid_blocks(a.NB) * a.KS_gu)),
                            dim3(MID_WAVES * 64), 0, s, a);
 }
 
