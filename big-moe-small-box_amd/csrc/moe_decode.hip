@@ -494,33 +494,81 @@ __global__ __launch_bounds__(GV_THREADS) void k_gu_epi(GvArgs a)
     *reinterpret_cast<u32x4*>(a.act_rows + (size_t)r * a.I + col) = pack8_r(act);
 }
 
-// Gate / up epilogue of row r, 128-column block cb, by one wave: its 128 fp16 down-input values go to dst (16 bytes per
-// lane of group 0, lane j at dst + 8 j: global memory or LDS). Lane group q = lane >> 4 loads splits q, q + 4, ... B at
-// a time (the sums are the same for every B) and the four groups' sums are added pairwise ((q0 + q1) + (q2 + q3)), so the k-splits cost one memory latency
-// instead of one per batch; the rest runs as in k_gu_epi (every group computes it, group 0 stores).
+// 128-point Hadamard over a wave whose lane 16 q + j holds elements 8 j + 2 q, 8 j + 2 q + 1: spans 2 and 4 between the
+// lane groups, 8 .. 64 inside the 16-lane rows. Same pairs, order and rounding as had128_wave.
+__device__ __forceinline__ void had128_q(float& v0, float& v1)
+{
+    const int lane = threadIdx.x & 63;
+    auto sgn = [&](int m) { return (lane & m) ? -1.0f : 1.0f; };
+    {
+        const float a = v0, b = v1;
+        v0 = a + b;
+        v1 = a - b;
+    }
+    v0 = __builtin_fmaf(sgn(16), v0, xor16_f(v0));
+    v1 = __builtin_fmaf(sgn(16), v1, xor16_f(v1));
+    v0 = __builtin_fmaf(sgn(32), v0, xor32_f(v0));
+    v1 = __builtin_fmaf(sgn(32), v1, xor32_f(v1));
+    v0 = __builtin_fmaf(sgn(1), v0, dpp_f<0xB1>(v0));
+    v1 = __builtin_fmaf(sgn(1), v1, dpp_f<0xB1>(v1));
+    v0 = __builtin_fmaf(sgn(2), v0, dpp_f<0x4E>(v0));
+    v1 = __builtin_fmaf(sgn(2), v1, dpp_f<0x4E>(v1));
+    v0 = __builtin_fmaf(sgn(4), v0, dpp_xor4(v0));
+    v1 = __builtin_fmaf(sgn(4), v1, dpp_xor4(v1));
+    v0 = __builtin_fmaf(sgn(8), v0, dpp_f<0x128>(v0));
+    v1 = __builtin_fmaf(sgn(8), v1, dpp_f<0x128>(v1));
+}
+
+// The sums over the four lane groups, ((q0 + q1) + (q2 + q3)), of v[0 .. 7]: group q gets those of v[2 q], v[2 q + 1].
+// permlane16_swap(x, y) puts x of both rows of a pair beside each other in the even row, y in the odd one.
+__device__ __forceinline__ void sum_groups_scatter(const float* v, float& s0, float& s1)
+{
+    auto bits = [](float f) { return __builtin_bit_cast(uint32_t, f); };
+    auto flt = [](uint32_t u) { return __builtin_bit_cast(float, u); };
+    float h[4];                                     // elements 0, 1, 4, 5 in even groups, 2, 3, 6, 7 in odd ones
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        const int e = (i & 1) + 4 * (i >> 1);
+        const auto r = __builtin_amdgcn_permlane16_swap(bits(v[e]), bits(v[e + 2]), false, false);
+        h[i] = flt(r[0]) + flt(r[1]);
+    }
+    const auto r0 = __builtin_amdgcn_permlane32_swap(bits(h[0]), bits(h[2]), false, false);
+    const auto r1 = __builtin_amdgcn_permlane32_swap(bits(h[1]), bits(h[3]), false, false);
+    s0 = flt(r0[0]) + flt(r0[1]);
+    s1 = flt(r1[0]) + flt(r1[1]);
+}
+
+// Gate / up epilogue of row r, 128-column block cb, by one wave: its 128 fp16 down-input values go to dst (4 bytes per
+// lane: global memory or LDS). Lane group q = lane >> 4 loads splits q, q + 4, ... B at a time (the sums are the same for
+// every B) and the four groups' sums are added pairwise ((q0 + q1) + (q2 + q3)), so the k-splits cost one memory latency
+// instead of one per batch. The addition leaves every lane two of the 128 columns (8 j + 2 q, + 1), and the rest runs as in
+// k_gu_epi on those: it is one wave's chain of dependent operations, and the activation, a fixed sequence of about 50 per
+// column, was half of it while every lane did eight columns. One token, 9 experts
+// of I 1536: the kernel 6.4 -> 4.9 us.
 template <int B>
 __device__ __forceinline__ void gu_epi_wave(const GvArgs& a, int r, int cb, uint16_t* dst)
 {
     const int lane = threadIdx.x & 63, q = lane >> 4, j = lane & 15;
     const int nrows = a.offsets[a.NE], e = a.row_expert[r];
-    const int col = cb * 128 + 8 * j;
+    const int col = 8 * j + 2 * q;
     // the row's scale vectors first: their chain of loads (expert record, then vectors) overlaps the split sums' loads
-    u32x4 svg4 = {0u, 0u, 0u, 0u}, svu4 = svg4, sud4 = svg4;
+    uint32_t svg = 0u, svu = 0u, sud = 0u;
     if (r < nrows)
     {
         const bmx_expert& ex = e == a.E ? *a.shared : a.experts[e];
-        svg4 = ldg4(reinterpret_cast<const uint16_t*>(ex.svh[0]) + col);
-        svu4 = ldg4(reinterpret_cast<const uint16_t*>(ex.svh[1]) + col);
-        sud4 = ldg4(reinterpret_cast<const uint16_t*>(ex.suh[2]) + col);
+        svg = ldg(reinterpret_cast<const uint16_t*>(ex.svh[0]) + cb * 128 + col, 0);
+        svu = ldg(reinterpret_cast<const uint16_t*>(ex.svh[1]) + cb * 128 + col, 0);
+        sud = ldg(reinterpret_cast<const uint16_t*>(ex.suh[2]) + cb * 128 + col, 0);
     }
-    float g[8], v[8];
+    float g0, g1, u0, u1;
     if (a.gu_half)
     {
-        // one fp16 split: every lane group loads the same values
-        const uint16_t* hp = reinterpret_cast<const uint16_t*>(a.part_gu) + ((size_t)r * a.NB + cb) * 256 + 8 * j;
-        unpack8(ldg4(hp), g);
-        unpack8(ldg4(hp + 128), v);
+        // one fp16 split
+        const uint16_t* hp = reinterpret_cast<const uint16_t*>(a.part_gu) + ((size_t)r * a.NB + cb) * 256 + col;
+        const uint32_t gw = ldg(hp, 0), uw = ldg(hp + 128, 0);
         if (r >= nrows) return;
+        g0 = h2f(gw & 0xffffu); g1 = h2f(gw >> 16); u0 = h2f(uw & 0xffffu); u1 = h2f(uw >> 16);
     }
     else
     {
@@ -529,32 +577,24 @@ __device__ __forceinline__ void gu_epi_wave(const GvArgs& a, int r, int cb, uint
         float gu[16];
         const int ks = r < nrows ? row_splits<false>(a, r) : a.KS_gu;
         sum_splits_short<4, B>(p, 4 * stride, (ks - q + 3) / 4, gu);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) gu[i] = gu[i] + xor16_f(gu[i]);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) gu[i] = gu[i] + xor32_f(gu[i]);
         if (r >= nrows) return;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) { g[i] = h2f(f2h_r(gu[i])); v[i] = h2f(f2h_r(gu[8 + i])); }
+        sum_groups_scatter(gu, g0, g1);
+        sum_groups_scatter(gu + 8, u0, u1);
+        g0 = h2f(f2h_r(g0)); g1 = h2f(f2h_r(g1)); u0 = h2f(f2h_r(u0)); u1 = h2f(f2h_r(u1));
     }
-    had128_x8(g);
-    had128_x8(v);
-    const float rs = R_SCALE * had128_x8_sign();      // the transforms' lane sign folded into the scale
-    float svg[8], svu[8], sud[8];
-    unpack8(svg4, svg);
-    unpack8(svu4, svu);
-    unpack8(sud4, sud);
-    float act[8];
+    had128_q(g0, g1);
+    had128_q(u0, u1);
+    float act[2];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 2; ++i)
     {
-        const float gi = (g[i] * rs) * svg[i], ui = (v[i] * rs) * svu[i];
-        act[i] = act_gate(a.act, a.gated, gi, ui, a.limit) * sud[i];
+        const int sh = 16 * i;
+        const float gi = ((i ? g1 : g0) * R_SCALE) * h2f((svg >> sh) & 0xffffu), ui = ((i ? u1 : u0) * R_SCALE) * h2f((svu >> sh) & 0xffffu);
+        act[i] = act_gate(a.act, a.gated, gi, ui, a.limit) * h2f((sud >> sh) & 0xffffu);
     }
-    had128_x8(act);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) act[i] = act[i] * rs;
-    if (q == 0) *reinterpret_cast<u32x4*>(dst + 8 * j) = pack8_r(act);
+    had128_q(act[0], act[1]);
+    *reinterpret_cast<uint32_t*>(dst + col) =
+        (uint32_t)f2h_r(act[0] * R_SCALE) | ((uint32_t)f2h_r(act[1] * R_SCALE) << 16);
 }
 
 // Small launches: one wave per (row, 128-column block).
@@ -1065,11 +1105,13 @@ int launch_decode_experts(const MoeShape& m, const void* x, const bmx_routes* r,
     a.filter = 0;
     // One-row groups (one token) with the activation and the down product in the same call and no act rows asked
     // for: the down GEMV computes the activation of its k-range itself, once per output block instead of once, for
-    // one launch and one round trip through memory fewer. Worth it up to 16 output blocks (H <= 2048: 31.0 -> 29.6 us
-    // for a 64-expert top-8 layer of H 2048, I 768); at 32 blocks the repeated epilogue costs what it saves.
+    // one launch and one round trip through memory fewer. Worth it while the down workgroups start in one round (5 per
+    // compute unit), so the repeated epilogues run side by side: 9 experts of H 4096, I 1536 (1,152 workgroups) 46.7 ->
+    // 44.8 us; in two rounds (7 experts of H 5120, I 2304: 1,680) it costs 64.8 -> 66.5.
     a.gu_half = 0;
     a.act_in_down = rows_per_group_of(m.T) == 1 && (stages & (1 << BMX_STAGE_ACT)) && (stages & (1 << BMX_STAGE_DOWN)) &&
-                    !act_rows && m.H / 128 <= 16 && act_in_down_allowed();
+                    !act_rows && (m.H / 128 <= 16 || (long)p.G_max * p.NBH * p.KS_dn <= 5L * cu_count()) &&
+                    act_in_down_allowed();
     switch (rows_per_group_of(m.T))
     {
         case 1: launch_mr<1>(a, q, stages, s, rf); break;
