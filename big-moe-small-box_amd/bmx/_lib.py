@@ -106,6 +106,7 @@ SIGNATURES = {
     "bmx_slot_prefetch_agent": (_I, [ctypes.POINTER(SlotTable), _P, _I, _P, _I, _I64, _I, ctypes.POINTER(_I64), _P]),
     "bmx_copy_wait": (_I, [_P, _I64, _I, _P]),
     "bmx_copy_wait_layer": (_I, [_P, _I, _I, _P]),
+    "bmx_moe_slots_forward": (_I, [ctypes.POINTER(MoeDesc), _P, _I, _P, _I, _P, _P, _P, _P, _SZ, _I, _P]),
     "bmx_cpu_expert_rows": (_I, [ctypes.POINTER(CpuExpert), _I, _I, _P, _I, _I, _I, _I, _I, _I, ctypes.c_float, _P, _I]),
     "bmx_cpu_expert_rows_fast": (_I, [ctypes.POINTER(CpuExpert), _I, _I, _P, _I, _I, _I, ctypes.c_float, _P, _I]),
     "bmx_decode_splits": (_I, [ctypes.POINTER(MoeDesc), _I, ctypes.POINTER(_I), ctypes.POINTER(_I), ctypes.POINTER(_I)]),

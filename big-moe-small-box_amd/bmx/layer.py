@@ -149,6 +149,18 @@ class MoELayer:
         the combine."""
         T, lib = x.shape[0], L.lib()
         desc = self.slot_desc
+        if self.slots.agent is not None or self.slots.copied[self.li] is None:
+            # the whole sequence in one library call; the copies to wait for are the copy agent's (or there are none)
+            self.slots.check()
+            need = lib.bmx_moe_workspace(desc, T, path)
+            if self._ws is None or self._ws.numel() < need:
+                self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+            out = torch.empty((T, self.hidden_size), dtype=torch.float32, device=x.device)
+            L.check(lib.bmx_moe_slots_forward(desc, self.slots.agent if self.slots.seq[self.li] else None, self.li,
+                                              x.data_ptr(), T, sel.data_ptr(), rw.data_ptr(), out.data_ptr(),
+                                              self._ws.data_ptr(), self._ws.numel(), path,
+                                              torch.cuda.current_stream().cuda_stream), "bmx_moe_slots_forward")
+            return out
         routes = ops.dispatch(sel, self.num_local_experts, self.routing_first, self.table.has_shared,
                               lib.bmx_rows_per_group(T, self.num_experts_per_tok, path))
         need = lib.bmx_experts_workspace(ctypes.byref(desc), T, path)
@@ -171,7 +183,6 @@ class MoELayer:
         self.slots.wait_copies(self.li, part="down")
         stage(L.STAGE_DOWN_STAGED)
         stage(L.STAGE_COMBINE)
-        self._routes = routes
         return out
 
     # ---- single-expert paths ----

@@ -42,6 +42,12 @@ int launch_dispatch(const int64_t* sel, int T, int topk, int E, int64_t first, i
 int groups_max(int T, int topk, int E, int shared, int rows_per_group);
 
 // moe_decode.hip
+// a one-token call's picks and the dispatch arrays its resident gate / up stage writes from them
+struct PickFuse {
+    const int64_t* sel;
+    int64_t first;
+    bmx_routes r;
+};
 struct MoeShape {
     int H, I, E, topk, T, shared, act, gated;
     float limit;
@@ -61,7 +67,7 @@ size_t decode_ws_bytes(const MoeShape& m);
 // ws layout: [part_gu][part_dn][act rows (used when act_rows == NULL)]; stages: 1 = gate/up, 2 = down (+ combine)
 int launch_decode_experts(const MoeShape& m, const void* x, const bmx_routes* r, float* y_rows, void* act_rows,
                           void* ws, size_t ws_bytes, float* combine_out, const void* combine_w, hipStream_t s, int stages,
-                          const RouteFuse* rf = nullptr);
+                          const RouteFuse* rf = nullptr, const PickFuse* pf = nullptr);
 int decode_rows_per_group(int T);
 // split path (BMX_PATH_SPLIT): the decode GEMVs for experts with few rows, the mid-size MFMA GEMMs for experts with at
 // least split_min_rows() rows, in one call; ws layout [part_gu][part_dn][act rows][xt]

@@ -377,6 +377,51 @@ int bmx_moe_forward(const bmx_moe_desc* desc, const void* x_fp16, int T, const i
     return launch_experts(p, m, x_fp16, &r, nullptr, nullptr, ews, ews_bytes, out, w_fp16, s, STAGES_LAYER);
 }
 
+int bmx_moe_slots_forward(const bmx_moe_desc* desc, bmx_copy_agent* agent, int li, const void* x_fp16, int T,
+                          const int64_t* sel, const void* w_fp16, float* out, void* workspace, size_t workspace_bytes,
+                          int path, bmx_stream_t stream)
+{
+    const char* fn = "bmx_moe_slots_forward";
+    int rc = check_desc(desc, fn);
+    if (rc) return rc;
+    const int p = resolve_path(path, T, desc->topk);
+    if (p < 0 || T < 0) return set_error(BMX_ERR_ARG, "%s: bad path %d or T %d", fn, path, T);
+    if (!desc->fresh) return set_error(BMX_ERR_ARG, "%s: needs desc->fresh", fn);
+    if (T == 0) return BMX_OK;
+    if (!x_fp16 || !sel || !w_fp16 || !out || !workspace) return set_error(BMX_ERR_ARG, "%s: null pointer", fn);
+    const size_t need = bmx_moe_workspace(desc, T, path);
+    if (workspace_bytes < need) return set_error(BMX_ERR_WORKSPACE, "%s: workspace %zu < %zu", fn, workspace_bytes, need);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const MoeShape m = shape_of(desc, T);
+    const int rpg = path_rows_per_group(p, T);
+    const RoutesLayout L = routes_layout(T, desc->topk, desc->E, m.shared, rpg);
+    char* base = static_cast<char*>(workspace);
+    PickFuse pf;
+    pf.sel = sel;
+    pf.first = desc->first;
+    pf.r = routes_at(base, L);
+    char* dws = base + L.total;
+    const size_t dws_bytes = align_up(dispatch_ws_bytes(T, desc->topk, desc->E), 256);
+    char* ews = dws + dws_bytes;
+    const size_t ews_bytes = align_up(experts_ws_bytes(p, m), 256);
+    const bool one = p == BMX_PATH_DECODE && T == 1;
+    auto run = [&](int stages) {
+        return one ? launch_decode_experts(m, x_fp16, &pf.r, nullptr, nullptr, ews, ews_bytes, out, w_fp16, s, stages, nullptr, &pf)
+                   : launch_experts(p, m, x_fp16, &pf.r, nullptr, nullptr, ews, ews_bytes, out, w_fp16, s, stages);
+    };
+    if (!one)
+    {
+        rc = launch_dispatch(sel, T, desc->topk, desc->E, desc->first, m.shared, rpg, &pf.r, dws, dws_bytes, nullptr, 0, s);
+        if (rc) return rc;
+    }
+    rc = run((1 << BMX_STAGE_PREP) | (1 << BMX_STAGE_GATE_UP_RESIDENT));
+    if (!rc && agent) rc = bmx_copy_wait_layer(agent, li, 0, stream);
+    if (!rc) rc = run((1 << BMX_STAGE_GATE_UP_STAGED) | (1 << BMX_STAGE_ACT) | (1 << BMX_STAGE_DOWN_RESIDENT));
+    if (!rc && agent) rc = bmx_copy_wait_layer(agent, li, 1, stream);
+    if (!rc) rc = run((1 << BMX_STAGE_DOWN_STAGED) | (1 << BMX_STAGE_COMBINE));
+    return rc;
+}
+
 // the layer call's workspace: bmx_moe_forward's, then the projected logits [T][E] fp16 (used when no logits are given)
 size_t bmx_moe_layer_workspace(const bmx_moe_desc* desc, int T, int path)
 {

@@ -343,6 +343,13 @@ int bmx_copy_wait(bmx_copy_agent* agent, int64_t seq, int part, bmx_stream_t str
  * record when that step admitted experts, else the records before it (the prefetches its hits came from); the step
  * leaves the target on the device, so a layer whose experts are in place waits for nothing in flight. */
 int bmx_copy_wait_layer(bmx_copy_agent* agent, int li, int part, bmx_stream_t stream);
+/* bmx_moe_forward on layer li of a slot table (desc->fresh: its fresh flags) after the layer's step: the gate / up products
+ * of the resident experts, the wait for the admitted experts' gate / up parts (bmx_copy_wait_layer; none when agent is
+ * NULL), their products, the activation, the same for down, the combine. The results of bmx_dispatch and the bmx_moe_stage
+ * calls in that order, bit for bit; workspace: bmx_moe_workspace(desc, T, path) bytes. */
+int bmx_moe_slots_forward(const bmx_moe_desc* desc, bmx_copy_agent* agent, int li, const void* x_fp16, int T,
+                          const int64_t* sel, const void* w_fp16, float* out, void* workspace, size_t workspace_bytes,
+                          int path, bmx_stream_t stream);
 
 /* ---- CPU expert lane ----
  * One expert's y rows (fp32 [nr][H]: the down projection after svh, what BMX_STAGE_COMBINE sums in slot order) for nr

@@ -242,6 +242,33 @@ def test_layer_with_staged_experts_matches_resident(cuda, copies):
         slots.close()
 
 
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("picks", [(3, 9, 7, 1), (5, 5, 2, 5), (-1, 24, 6, 6), (30, -7, 24, 99), (0, 23, 23, 0)])
+def test_one_token_given_picks(cuda, picks, shared):
+    """A one-token slot-table call orders its picks itself (duplicates, ids out of range, no pick at all): the bits of the
+    resident layer's dispatch and products."""
+    import bmx
+    E, H, I, topk = 24, 512, 256, 4
+    tab = bmx.ExpertTable.random(H, I, E, (bmx.TF_K3, bmx.TF_K2, bmx.TF_K4), shared=shared, seed=21, device=cuda)
+    ref = bmx.MoELayer(tab, topk)
+    host = bmx.ExpertTable.random(H, I, E, (bmx.TF_K3, bmx.TF_K2, bmx.TF_K4), shared=shared, seed=21, device=cuda)
+    slots = bmx.ExpertSlots([host], 8, maxj=4, copies="dma")
+    m = bmx.MoELayer(host, topk, slots=slots)
+    g = torch.Generator(device=cuda)
+    g.manual_seed(22)
+    x = torch.randn((1, H), generator=g, device=cuda).half()
+    w = (torch.rand((1, topk), generator=g, device=cuda) + 0.2).half()
+    sel = torch.tensor([picks], dtype=torch.int64, device=cuda)
+    for step in range(2):                # admitted, then resident
+        sg, wg, _ = m.layer(0, sel, w, x, 1)
+        got = m.run_bszN(x, sg, wg)
+        want = ref.run_bszN(x, sel, w)
+        torch.cuda.synchronize()
+        say("given picks", picks, shared, step)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    slots.close()
+
+
 @pytest.mark.parametrize("copies", ["kernel", "dma"])
 def test_prefetch_keeps_outputs(cuda, copies):
     """A decode loop over a stack of layers with homes in pinned host memory, each layer's step followed by a prefetch
