@@ -525,6 +525,9 @@ __device__ __forceinline__ int ep_unit()
     return (blockIdx.x * GV_WAVES + (threadIdx.x >> 6)) * UPW + ((threadIdx.x & 63) >> 4);
 }
 constexpr long EP_SMALL = 16384;              // launches with fewer units use UPW = 1
+// The gate / up epilogue's own line: a wave per unit costs four times the activations of 16 lanes per unit, which shows once
+// the units fill the SIMDs (11,088 units, four splits: 16.8 us against 14.4)
+constexpr long EP_SMALL_GU = 4096;
 
 // gate / up epilogue: sum of the splits in split order -> fp16 gate / up (the stored GEMV / GEMM results) -> H128 * R * svh
 // -> activation -> * down suh -> H128 * R -> fp16 down-input row (exllamav3 kernel A epilogue order,
@@ -859,12 +862,18 @@ __global__ __launch_bounds__(GV_THREADS) void k_dn_combine(GvArgs a)
 
 // The combine of token t's 128-column block cb by one workgroup: 16-lane group k computes slot k (the shared expert's
 // row is slot topk) into ys[k], then group 0 sums them in slot order: the same sums in the same order as k_dn_combine.
-// ys: [topk + 1][128] floats and live: [topk + 1] ints of LDS.
+// ys: [topk + 1][128] floats and live: [topk + 2] ints of LDS. A gated shared expert's gate is computed beside the slots, by the
+// last group (a wave without slots up to 12 of them): 77 tokens, 33 -> 17 us with the gate's loads batched.
 constexpr int CB_MAXS = 33;
 __device__ __forceinline__ void combine_block(const GvArgs& a, int t, int cb, float (*ys)[128], int* live)
 {
     const int k0 = threadIdx.x >> 4, j = threadIdx.x & 15;
-    const int ns = a.topk + (a.has_shared ? 1 : 0);
+    const int ns = a.topk + (a.has_shared ? 1 : 0), gate = a.has_shared && a.sh_gate ? ns : -1;
+    if (gate >= 0 && k0 == GV_THREADS / 16 - 1)
+    {
+        const float g = shared_gate16(a.x + (size_t)t * a.H, a.sh_gate, a.H);
+        if (j == 0) live[gate] = __builtin_bit_cast(int, g);
+    }
     for (int k = k0; k < ns; k += GV_THREADS / 16)
     {
         int r;
@@ -888,7 +897,7 @@ __device__ __forceinline__ void combine_block(const GvArgs& a, int t, int cb, fl
     }
     lds_barrier();
     if (k0) return;
-    const float g = (a.has_shared && a.sh_gate) ? shared_gate16(a.x + (size_t)t * a.H, a.sh_gate, a.H) : 1.0f;
+    const float g = gate >= 0 ? __builtin_bit_cast(float, live[gate]) : 1.0f;
     float o[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = 0.0f;
@@ -920,7 +929,7 @@ __device__ __forceinline__ void combine_block(const GvArgs& a, int t, int cb, fl
 __global__ __launch_bounds__(GV_THREADS) void k_dn_combine_par(GvArgs a)
 {
     __shared__ float ys[CB_MAXS][128];
-    __shared__ int live[CB_MAXS];
+    __shared__ int live[CB_MAXS + 1];
     combine_block(a, blockIdx.x / a.NBH, blockIdx.x % a.NBH, ys, live);
 }
 
@@ -976,7 +985,7 @@ int launch_epilogue(const GvArgs& a, int stage, hipStream_t s)
     switch (stage)
     {
         case BMX_STAGE_ACT:
-            if (gu >= EP_SMALL) hipLaunchKernelGGL(k_gu_epi<4>, wgs(gu, 4), dim3(GV_THREADS), 0, s, a);
+            if (gu >= EP_SMALL_GU) hipLaunchKernelGGL(k_gu_epi<4>, wgs(gu, 4), dim3(GV_THREADS), 0, s, a);
             else hipLaunchKernelGGL(k_gu_epi_w, wgs(gu, 1), dim3(GV_THREADS), 0, s, a);
             break;
         case BMX_STAGE_COMBINE:
@@ -995,7 +1004,7 @@ int launch_epilogue(const GvArgs& a, int stage, hipStream_t s)
 int decode_gu_grouped(const MoeShape& m)
 {
     const DecodePlan p = decode_plan(m);
-    return (long)p.R_max * p.NB < EP_SMALL ? 1 : 0;     // k_gu_epi_w and the one-token down prologue: gu_epi_wave
+    return (long)p.R_max * p.NB < EP_SMALL_GU ? 1 : 0;     // k_gu_epi_w and the one-token down prologue: gu_epi_wave
 }
 
 // ---- plan ------------------------------------------------------------------------------------------------------------

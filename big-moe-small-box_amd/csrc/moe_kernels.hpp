@@ -72,16 +72,31 @@ __device__ __forceinline__ int row_splits(const GvArgs& a, int r)
 // the same on both lanes); then the fixed-sequence sigmoid. The oracle evaluates the same sequence.
 __device__ __forceinline__ float shared_gate16(const uint16_t* x, const uint16_t* g, int H)
 {
-    const int j = threadIdx.x & 15;
+    constexpr int U = 8;                  // blocks per round trip to memory
+    const int j = threadIdx.x & 15, nb = H / 128;
     float acc = 0.0f;
-    for (int b = 0; b < H / 128; ++b)
-    {
+    auto add = [&](const u32x4& xw, const u32x4& gw) {
         float xv[8], gv[8];
-        unpack8(ldg4(x + 128 * b + 8 * j), xv);
-        unpack8(ldg4(g + 128 * b + 8 * j), gv);
+        unpack8(xw, xv);
+        unpack8(gw, gv);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc = __builtin_fmaf(xv[i], gv[i], acc);
+    };
+    int b = 0;
+    for (; b + U <= nb; b += U)
+    {
+        u32x4 xw[U], gw[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            xw[u] = ldg4(x + 128 * (b + u) + 8 * j);
+            gw[u] = ldg4(g + 128 * (b + u) + 8 * j);
+        }
+        __builtin_amdgcn_sched_barrier(0);       // every load before the first sum
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(xw[u], gw[u]);
     }
+    for (; b < nb; ++b) add(ldg4(x + 128 * b + 8 * j), ldg4(g + 128 * b + 8 * j));
     acc = acc + dpp_f<0x128>(acc);     // lane ^ 8 (row_ror:8)
     acc = acc + dpp_xor4(acc);
     acc = acc + dpp_f<0x4E>(acc);      // lane ^ 2

@@ -629,14 +629,14 @@ struct MidPlan {
 // k-split: the most splits that keep at least min_steps k-steps of 64 each, gate / up (BMX_MID_MIN_STEPS) and down
 // (BMX_MID_MIN_STEPS_DN). Splits even out the SIMDs' shares (the routing, unknown here, may put all rows on a few experts),
 // at the price of partial sums that the epilogues add. Up to MID_FEW_ROWS dispatch rows the partials are small: 8 and 4
-// steps, above them 16 and 8. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60 experts of H 4096,
+// steps, above them 16. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60 experts of H 4096,
 // I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I 2048) 8 x 4: 86, 4 x 4:
-// 92, 16 x 4: 95, 16 x 16: 103; 77 tokens (693 rows, 255 experts) 16 x 8: 591, 8 x 8: 608, 16 x 4: 609, 32 x 8: 600.
+// 92, 16 x 4: 95, 16 x 16: 103; 77 tokens (693 rows, ~150 experts) 16 x 16: 547, 16 x 8: 560, 16 x 32: 549, 32 x 16: 561, 8 x 8: 608.
 constexpr int MID_FEW_ROWS = 160;
 static int mid_split(int ksteps, bool down, int rows)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
-    const int min_steps = (v && *v) ? atoi(v) : (rows <= MID_FEW_ROWS ? 8 : 16) / (down ? 2 : 1);
+    const int min_steps = (v && *v) ? atoi(v) : rows > MID_FEW_ROWS ? 16 : down ? 4 : 8;
     for (int d = ksteps; d > 1; --d)
         if (ksteps % d == 0 && ksteps / d >= min_steps) return d;
     return 1;
