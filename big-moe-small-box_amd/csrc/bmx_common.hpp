@@ -265,13 +265,12 @@ __device__ __forceinline__ u32x4 pack8_r(const float (&v)[8])
 // n = rint(x / ln 2), r = x - n ln 2 with ln 2 split into a high part of 17 significant bits and a low part (the split
 // SLEEF's expf uses: 0.693145751953125 + 1.428606765330187e-06); exp(r) by the Taylor polynomial of degree 7 in Horner
 // form (|r| <= ln 2 / 2); 2^n applied as two exact power-of-two factors, so a subnormal result rounds once.
+// Without branches (the ends of the range and NaN by selects), so that several of them run side by side.
 __device__ __forceinline__ float exp_fixed(float x)
 {
-    if (x != x) return x;
-    if (x > 88.72f) return __builtin_huge_valf();
-    if (x < -104.0f) return 0.0f;
-    const float n = __builtin_rintf(__fmul_rn(x, 1.44269504f));
-    float r = __builtin_fmaf(n, -0.693145751953125f, x);
+    const float xc = fminf(fmaxf(x, -104.0f), 88.72f);
+    const float n = __builtin_rintf(__fmul_rn(xc, 1.44269504f));
+    float r = __builtin_fmaf(n, -0.693145751953125f, xc);
     r = __builtin_fmaf(n, -1.428606765330187e-06f, r);
     float p = 1.98412698e-4f;
     p = __builtin_fmaf(p, r, 1.38888889e-3f);
@@ -285,7 +284,10 @@ __device__ __forceinline__ float exp_fixed(float x)
     const int n1 = ni / 2, n2 = ni - n1;
     const float s1 = __builtin_bit_cast(float, (uint32_t)(n1 + 127) << 23);
     const float s2 = __builtin_bit_cast(float, (uint32_t)(n2 + 127) << 23);
-    return __fmul_rn(__fmul_rn(p, s1), s2);
+    float v = __fmul_rn(__fmul_rn(p, s1), s2);
+    v = x > 88.72f ? __builtin_huge_valf() : v;
+    v = x < -104.0f ? 0.0f : v;
+    return x != x ? x : v;
 }
 
 __device__ __forceinline__ float sigmoid_fixed(float x)
