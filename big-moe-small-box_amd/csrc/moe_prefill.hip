@@ -632,13 +632,17 @@ struct MidPlan {
 // steps, above them 16. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60 experts of H 4096,
 // I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I 2048) 8 x 4: 86, 4 x 4:
 // 92, 16 x 4: 95, 16 x 16: 103; 77 tokens (693 rows, ~150 experts) 16 x 16: 547, 16 x 8: 560, 16 x 32: 549, 32 x 16: 561, 8 x 8: 608.
+// A matrix's partials past MID_FEW_BYTES keep the 16 steps, so no call outgrows bmx_moe_layer_scratch by them.
 constexpr int MID_FEW_ROWS = 160;
-static int mid_split(int ksteps, bool down, int rows)
+constexpr size_t MID_FEW_BYTES = 12u << 20;
+static int mid_split(int ksteps, bool down, int rows, size_t split_bytes)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
-    const int min_steps = (v && *v) ? atoi(v) : rows > MID_FEW_ROWS ? 16 : down ? 4 : 8;
+    const int min_steps = (v && *v) ? atoi(v) : 16, few_steps = down ? 4 : 8;
+    const bool few = !(v && *v) && rows <= MID_FEW_ROWS;
     for (int d = ksteps; d > 1; --d)
-        if (ksteps % d == 0 && ksteps / d >= min_steps) return d;
+        if (ksteps % d == 0 && (ksteps / d >= min_steps || (few && ksteps / d >= few_steps && d * split_bytes <= MID_FEW_BYTES)))
+            return d;
     return 1;
 }
 
@@ -649,8 +653,8 @@ static MidPlan mid_plan(const MoeShape& m)
     p.NBH = m.H / 128;
     p.G_max = groups_max(m.T, m.topk, m.E, m.shared, MID_M);
     p.R_max = m.T * m.topk + (m.shared ? m.T : 0);
-    p.KS_gu = mid_split(m.H / 64, false, p.R_max);
-    p.KS_dn = mid_split(m.I / 64, true, p.R_max);
+    p.KS_gu = mid_split(m.H / 64, false, p.R_max, (size_t)p.R_max * p.NB * 1024);
+    p.KS_dn = mid_split(m.I / 64, true, p.R_max, (size_t)p.R_max * p.NBH * 512);
     p.xt_bytes = (size_t)2 * p.R_max * m.H * 2;
     p.part_gu_bytes = (size_t)p.KS_gu * p.R_max * p.NB * 256 * 4;
     p.act_bytes = (size_t)p.R_max * m.I * 2;
