@@ -1056,6 +1056,15 @@ DecodePlan decode_plan(const MoeShape& m)
     // the staged input rows (NM matrices x MR rows x k-range fp16) must fit GV_LDS_X
     const int max_kr_gu = GV_LDS_X / (2 * MR * 2), max_kr_dn = GV_LDS_X / (MR * 2);
     int ks = pick_split(m.H / 128, est * p.NB, target_wgs(), "BMX_KS_GU");
+    if (MR > 1)
+    {
+        // several tokens: four workgroups start per compute unit, so just over 1,024 of them run as two rounds, the second
+        // nearly empty; twice the target unless a split would get under 256 of k (its rotation and start then cost more: 4
+        // tokens of H 2048 46.4 -> 47.6 us). H 4096, 9 experts a token: 2 tokens 75.3 -> 73.8, 3 tokens 107 -> 98.5, 4 tokens
+        // 124.9 -> 121.0; with 6 experts and I 2048, 4 tokens 103.1 -> 99.3
+        const int k2 = pick_split(m.H / 128, est * p.NB, 2 * target_wgs(), "BMX_KS_GU");
+        if (m.H / k2 >= 256) ks = k2;
+    }
     while (m.H / ks > max_kr_gu) { int d = ks + 1; while ((m.H / 128) % d) ++d; ks = d; }
     p.KS_gu = ks;
     ks = pick_split(m.I / 128, est * p.NBH, target_wgs(), "BMX_KS_DN");

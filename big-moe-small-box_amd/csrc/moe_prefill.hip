@@ -3,9 +3,9 @@
 // accumulation; each output element is one fixed sum (k ascending in MFMA blocks), independent of scheduling.
 //
 //   k_pf_prep_tok : rotated gate / up inputs of every dispatch row, xt = RN16(H128(x * suh) * R), token-major
-//   k_pf_gemm<false> : gate or up products of one 512-column block -> fp16 [row][128-block][gate | up][128]
+//   k_pf_gemm<false> : gate or up products of one 256-column block -> fp16 [row][128-block][gate | up][128]
 //   (k_gu_epi)    : fp16 gate / up -> epilogue -> fp16 down-input rows (shared with the decode path)
-//   k_pf_gemm<true>  : down products of one 512-column block -> fp32 [row][128-block][128]
+//   k_pf_gemm<true>  : down products of one 256-column block -> fp32 [row][128-block][128]
 //   (k_dn_combine): rotation * svh, slots summed in slot order (shared with the decode path)
 #include "moe_kernels.hpp"
 
@@ -123,16 +123,18 @@ __device__ __forceinline__ void step_barrier()
 }
 
 // ---- grouped GEMM ----------------------------------------------------------------------------------------------------
-// Work unit: (group of <= 128 rows, matrix, 512-column block); 8 waves, two per SIMD, all alike. Wave w owns the columns
-// of parity w & 1 (strip half) of 128-column block w >> 1, all rows of the group, and decodes its weights straight into
-// the B operand registers of v_mfma_f32_32x32x16_f16: lane L holds the strip of tile-row L / 32 of a pair of tile-rows
+// Work unit: (group of <= 128 rows, matrix, 256-column block); 4 waves, all alike, two workgroups per CU. Wave w owns the
+// columns of parity w & 1 (strip half) of 128-column block w >> 1, all rows of the group, and decodes its weights straight
+// into the B operand registers of v_mfma_f32_32x32x16_f16: lane L holds the strip of tile-row L / 32 of a pair of tile-rows
 // (32 k), so an operand's k index 8 (L / 32) + j is input row 8 q + j of that tile-row (q: the strip's upper or lower
 // eight rows), and its column is the lane's strip column. No B fragment passes through the LDS, and no weight is decoded
-// twice in a workgroup. The A rows (128 k at a time) are staged in LDS in operand order and shared by the 8 waves.
-// What bounds it: MFMA (16 per 32 k and wave at 128 rows, 512 cycles) and the decode (115 VALU, 460 cycles) of two waves
-// overlap on a SIMD; the chip then runs into its power limit (the shader clock falls to 1.6-1.8 GHz). Against four MFMA
-// and eight decode waves handing B over through LDS: layer of 8,192 tokens (384 experts, top-6, H 4096, I 2048, K 2 / 3)
-// 5,008 -> 4,427 us, of 517 tokens 1,878 -> 1,433, of 2,048 tokens (H 5120, I 2304, K 2.5 / 2) 3,612 -> 2,959.
+// twice in a workgroup. The A rows (64 k at a time) are staged in LDS in operand order and shared by the 4 waves.
+// What bounds it: the decode (115 VALU per 32 k and wave) and the MFMAs (16 at 128 rows) of two waves overlap on a SIMD, and
+// the chip then runs into its power limit (the shader clock falls to 1.7-1.9 GHz, VALU 0.7 busy, MFMA 0.45). Layer times, four
+// MFMA and eight decode waves handing B over through LDS -> eight equal waves of 512 columns -> decode and products
+// interleaved -> this: 8,192 tokens (384 experts, top-6, H 4096, I 2048, K 2 / 3) 5,008 -> 4,427 -> 4,192 -> 4,135 us; 517
+// tokens 1,878 -> 1,433 -> 1,401 -> 1,336; 2,048 tokens (H 5120, I 2304, K 2.5 / 2) 3,612 -> 2,959 -> 2,903 -> 2,755. Units of
+// at most 32 rows without stages and barriers, as the mid-size kernel runs them: the same time (the clock is the limit).
 // The scheduling fences keep a pair's operand reads, decode and products apart: the compiler otherwise moves two pairs'
 // decodes together and spills.
 constexpr int PF_WAVES = 4;
