@@ -113,6 +113,13 @@ class MoELayer:
                                        first=self.routing_first)
         return sel, w, False
 
+    def _workspace(self, need):
+        """The layer's workspace, at least need bytes. On the table's device whatever the call's tensors are on: a call
+        that is refused for a host tensor leaves no host memory behind for the next one to hand to the kernels."""
+        if self._ws is None or self._ws.numel() < need:
+            self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=self.table.device)
+        return self._ws
+
     # ---- experts + combine ----
     def run_bszN(self, z, sel, rw, path=L.PATH_AUTO):
         x = z.view(-1, self.hidden_size)
@@ -128,8 +135,7 @@ class MoELayer:
         if self.slots is not None and staged is not None:
             # every expert's table entry points at a slot or at the staging arena: the plain layer, then the restore
             need = L.lib().bmx_moe_workspace(self.slot_desc, x.shape[0], path)
-            if self._ws is None or self._ws.numel() < need:
-                self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+            self._workspace(need)
             self.out_bszn = ops.moe_forward(self.slot_desc, x, sel, rw, path, self._ws)
             self.slots.stage_restore(staged)
             return self.out_bszn
@@ -137,8 +143,7 @@ class MoELayer:
             self.out_bszn = self._run_slots(x, sel, rw, path)
             return self.out_bszn
         need = L.lib().bmx_moe_workspace(self.desc, x.shape[0], path)
-        if self._ws is None or self._ws.numel() < need:
-            self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+        self._workspace(need)
         self.out_bszn = ops.moe_forward(self.desc, x, sel, rw, path, self._ws)
         return self.out_bszn
 
@@ -153,8 +158,7 @@ class MoELayer:
             # the whole sequence in one library call; the copies to wait for are the copy agent's (or there are none)
             self.slots.check()
             need = lib.bmx_moe_workspace(desc, T, path)
-            if self._ws is None or self._ws.numel() < need:
-                self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+            self._workspace(need)
             out = torch.empty((T, self.hidden_size), dtype=torch.float32, device=x.device)
             L.check(lib.bmx_moe_slots_forward(desc, self.slots.agent if self.slots.seq[self.li] else None, self.li,
                                               x.data_ptr(), T, sel.data_ptr(), rw.data_ptr(), out.data_ptr(),
@@ -164,8 +168,7 @@ class MoELayer:
         routes = ops.dispatch(sel, self.num_local_experts, self.routing_first, self.table.has_shared,
                               lib.bmx_rows_per_group(T, self.num_experts_per_tok, path))
         need = lib.bmx_experts_workspace(ctypes.byref(desc), T, path)
-        if self._ws is None or self._ws.numel() < need:
-            self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+        self._workspace(need)
         out = torch.empty((T, self.hidden_size), dtype=torch.float32, device=x.device)
         s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         P = lambda t: ctypes.c_void_p(t.data_ptr())
@@ -268,8 +271,7 @@ class MoELayer:
                 x = x.half().contiguous()
             lg = logits.view(x.shape[0], -1).to(torch.float16).contiguous() if logits is not None else None
             need = L.lib().bmx_moe_layer_workspace(self.desc, x.shape[0], path)
-            if self._ws is None or self._ws.numel() < need:
-                self._ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+            self._workspace(need)
             out, self.sel, self.w = ops.moe_layer(self.desc, self.router, x, lg, path, self._ws)
             self.out_bszn = out
             return out

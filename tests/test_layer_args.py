@@ -1,0 +1,32 @@
+"""Layer calls refuse host tensors before anything is enqueued, and a refused call leaves the layer as it was (CPU only)."""
+import types
+
+import pytest
+import torch
+
+
+def bare_layer(slots=None, topk=4):
+    """A MoELayer as its argument checks see it: no device memory behind it (its table is on the meta device)."""
+    import bmx
+    m = bmx.MoELayer.__new__(bmx.MoELayer)
+    m.num_experts_per_tok, m.num_local_experts, m.routing_first = topk, 8, 0
+    m.hidden_size, m.intermediate_size = 256, 128
+    m.table = types.SimpleNamespace(has_shared=False, device=torch.device("meta"))
+    m.slots, m.li, m._ws, m._staged, m.router_weight, m.router = slots, 0, None, None, None, bmx._lib.RouterDesc()
+    m.desc = m.slot_desc = bmx._lib.MoeDesc(256, 128, 8, topk, 0, 0, 1, 0.0, 16, None, 32)
+    return m
+
+
+def host_call(T):
+    return torch.zeros((T, 256)).half(), torch.zeros((T, 4), dtype=torch.int64), torch.ones((T, 4)).half()
+
+
+@pytest.mark.parametrize("T", [1, 3])
+def test_refused_call_keeps_no_host_workspace(T):
+    """The workspace a refused call leaves behind is the next call's: never host memory."""
+    m = bare_layer()
+    x, sel, w = host_call(T)
+    for call in (lambda: m.run_bszN(x, sel, w), lambda: m.forward(x, torch.zeros((T, 8)).half())):
+        with pytest.raises(ValueError, match="device tensor"):
+            call()
+        assert m._ws is None or m._ws.device.type != "cpu"
