@@ -157,14 +157,9 @@ class MoELayer:
         if self.slots.agent is not None or self.slots.copied[self.li] is None:
             # the whole sequence in one library call; the copies to wait for are the copy agent's (or there are none)
             self.slots.check()
-            need = lib.bmx_moe_workspace(desc, T, path)
-            self._workspace(need)
-            out = torch.empty((T, self.hidden_size), dtype=torch.float32, device=x.device)
-            L.check(lib.bmx_moe_slots_forward(desc, self.slots.agent if self.slots.seq[self.li] else None, self.li,
-                                              x.data_ptr(), T, sel.data_ptr(), rw.data_ptr(), out.data_ptr(),
-                                              self._ws.data_ptr(), self._ws.numel(), path,
-                                              torch.cuda.current_stream().cuda_stream), "bmx_moe_slots_forward")
-            return out
+            self._workspace(lib.bmx_moe_workspace(desc, T, path))
+            return ops.moe_slots_forward(desc, self.slots.agent if self.slots.seq[self.li] else None, self.li, x, sel, rw,
+                                         path, self._ws)
         routes = ops.dispatch(sel, self.num_local_experts, self.routing_first, self.table.has_shared,
                               lib.bmx_rows_per_group(T, self.num_experts_per_tok, path))
         need = lib.bmx_experts_workspace(ctypes.byref(desc), T, path)

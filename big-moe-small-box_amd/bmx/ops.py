@@ -134,6 +134,28 @@ def moe_forward(desc, x, sel, w, path=L.PATH_AUTO, workspace=None):
     return out
 
 
+def moe_slots_forward(desc, agent, li, x, sel, w, path=L.PATH_AUTO, workspace=None):
+    """moe_forward on layer li of a slot table after the layer's step (bmx_moe_slots_forward); agent: the copy agent whose
+    copies the layer's products wait for, or None."""
+    _need(x, torch.float16, "x"); _need(sel, torch.int64, "sel"); _need(w, torch.float16, "w")
+    T = x.shape[0]
+    if tuple(x.shape) != (T, desc.H) or tuple(sel.shape) != (T, desc.topk) or tuple(w.shape) != (T, desc.topk):
+        raise ValueError(f"moe_slots_forward: x {tuple(x.shape)}, sel {tuple(sel.shape)}, w {tuple(w.shape)} are not "
+                         f"[T, {desc.H}] and [T, {desc.topk}] of one T")
+    out = torch.empty((T, desc.H), dtype=torch.float32, device=x.device)
+    if T == 0:
+        return out
+    need = lib().bmx_moe_workspace(desc, T, path)
+    if need == 0:
+        check(1, "bmx_moe_workspace")
+    if workspace is None or workspace.numel() < need:
+        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    check(lib().bmx_moe_slots_forward(desc, agent, li, x.data_ptr(), T, sel.data_ptr(), w.data_ptr(), out.data_ptr(),
+                                      workspace.data_ptr(), workspace.numel(), path,
+                                      torch.cuda.current_stream().cuda_stream), "bmx_moe_slots_forward")
+    return out
+
+
 def moe_experts(desc, x, routes, path=L.PATH_AUTO, with_act=False):
     """Expert products on given routes -> (y_rows fp32 [R, H], act_rows fp16 [R, I] or None)."""
     T = x.shape[0]

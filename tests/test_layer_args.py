@@ -30,3 +30,32 @@ def test_refused_call_keeps_no_host_workspace(T):
         with pytest.raises(ValueError, match="device tensor"):
             call()
         assert m._ws is None or m._ws.device.type != "cpu"
+
+
+@pytest.mark.parametrize("T", [1, 3])
+def test_slot_call_refuses_host_tensors(T):
+    """A slot-table call with a host selection (host rows, host weights) raises: a kernel would read host addresses."""
+    m = bare_layer(types.SimpleNamespace(agent=None, copied=[None], seq=[0], check=lambda: None))
+    with pytest.raises(ValueError, match="device tensor"):
+        m.run_bszN(*host_call(T))
+
+
+class Dev:
+    """Stands for a contiguous device tensor of a shape (the checks read nothing else)."""
+    is_cuda, device = True, "cuda:0"
+
+    def __init__(self, shape, dtype):
+        self.shape, self.dtype = shape, dtype
+
+    def is_contiguous(self):
+        return True
+
+
+@pytest.mark.parametrize("xs,ss,ws", [((2, 256), (2, 3), (2, 4)), ((2, 256), (2, 5), (2, 5)), ((2, 256), (1, 4), (2, 4)),
+                                      ((2, 256), (2, 4), (2, 3)), ((2, 128), (2, 4), (2, 4)), ((2, 256), (8,), (2, 4))])
+def test_slot_call_refuses_other_shapes(xs, ss, ws):
+    """Picks or weights that are not the call's T rows of topk, or rows that are not H long, would be read out of range."""
+    import bmx
+    x, sel, w = Dev(xs, torch.float16), Dev(ss, torch.int64), Dev(ws, torch.float16)
+    with pytest.raises(ValueError, match="of one T"):
+        bmx.ops.moe_slots_forward(bare_layer().slot_desc, None, 0, x, sel, w)
