@@ -534,6 +534,12 @@ static hsa_status_t find_agents(hsa_agent_t ag, void* data)
     return HSA_STATUS_SUCCESS;
 }
 
+int check_agent_layer(const bmx_copy_agent* a, int li, const char* who)
+{
+    if (li < 0 || li >= a->t.L) return set_error(BMX_ERR_ARG, "%s: bad layer %d", who, li);
+    return BMX_OK;
+}
+
 }  // namespace bmx
 
 using namespace bmx;
@@ -861,8 +867,8 @@ int bmx_copy_wait(bmx_copy_agent* a, int64_t seq, int part, bmx_stream_t stream)
 int bmx_copy_wait_layer(bmx_copy_agent* a, int li, int part, bmx_stream_t stream)
 {
     if (!a) return set_error(BMX_ERR_ARG, "bmx_copy_wait_layer: null agent");
-    if (part < 0 || part > 1 || li < 0 || li >= a->t.L)
-        return set_error(BMX_ERR_ARG, "bmx_copy_wait_layer: bad part %d or layer %d", part, li);
+    if (part < 0 || part > 1) return set_error(BMX_ERR_ARG, "bmx_copy_wait_layer: bad part %d", part);
+    if (const int rc = check_agent_layer(a, li, "bmx_copy_wait_layer")) return rc;
     hipLaunchKernelGGL(k_copy_wait, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), a->sh_dev, part, (int64_t)0,
                        a->need + li, a->wait_ticks);
     return check_launch("bmx_copy_wait_layer");

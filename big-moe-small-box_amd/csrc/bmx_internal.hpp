@@ -151,6 +151,9 @@ int launch_slot_prefetch(const bmx_slot_table* t, int li, const int64_t* sel, in
                          hipStream_t s, AgentShared* sh = nullptr, int64_t seq = 0, int64_t wait_limit = 0);
 int launch_slot_copy(const bmx_slot_table* t, int li, int mats, int buf, hipStream_t s);
 
+// agent.hip
+int check_agent_layer(const bmx_copy_agent* a, int li, const char* who);
+
 // moe_prefill.hip (same ws / stage conventions; ws layout [xt][part_gu][act rows][part_dn])
 int prefill_rows_per_group();
 int mid_rows_per_group();

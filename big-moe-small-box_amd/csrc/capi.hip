@@ -387,6 +387,7 @@ int bmx_moe_slots_forward(const bmx_moe_desc* desc, bmx_copy_agent* agent, int l
     const int p = resolve_path(path, T, desc->topk);
     if (p < 0 || T < 0) return set_error(BMX_ERR_ARG, "%s: bad path %d or T %d", fn, path, T);
     if (!desc->fresh) return set_error(BMX_ERR_ARG, "%s: needs desc->fresh", fn);
+    if (agent && (rc = check_agent_layer(agent, li, fn))) return rc;      // here, not at the first wait: half is enqueued then
     if (T == 0) return BMX_OK;
     if (!x_fp16 || !sel || !w_fp16 || !out || !workspace) return set_error(BMX_ERR_ARG, "%s: null pointer", fn);
     const size_t need = bmx_moe_workspace(desc, T, path);

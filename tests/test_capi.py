@@ -134,3 +134,28 @@ def test_route_slot_step_checks():
     assert call(t, E=48) == B.BMX_ERR_ARG and b"not the table's" in L.bmx_last_error()
     assert call(t, topk=41) == B.BMX_ERR_ARG and b"unsupported sizes" in L.bmx_last_error()
     assert call(t, n_group=3) == B.BMX_ERR_ARG and b"bad groups" in L.bmx_last_error()
+
+
+def test_moe_slots_forward_checks():
+    """bmx_moe_slots_forward refuses bad descriptors, paths, token counts, pointers and workspaces before any device work;
+    a zero-token call does nothing."""
+    import bmx
+    B = bmx._lib
+    L = bmx.lib()
+    p = [ctypes.c_void_p(256 * (i + 1)) for i in range(5)]
+
+    def call(T=1, fresh=True, H=4096, path=0, x=p[0], sel=p[1], w=p[2], out=p[3], ws=p[4], n=1 << 40):
+        d = B.MoeDesc(H, 1536, 288, 8, 0, 0, 1, 0.0, ctypes.c_void_p(16), None, ctypes.c_void_p(32) if fresh else None)
+        return L.bmx_moe_slots_forward(ctypes.byref(d), None, 0, x, T, sel, w, out, ws, n, path, None)
+
+    assert call(H=100) == B.BMX_ERR_ARG and b"multiples of 128" in L.bmx_last_error()
+    assert call(path=7) == B.BMX_ERR_ARG and b"bad path" in L.bmx_last_error()
+    assert call(T=-1) == B.BMX_ERR_ARG and b"T -1" in L.bmx_last_error()
+    assert call(fresh=False) == B.BMX_ERR_ARG and b"desc->fresh" in L.bmx_last_error()
+    for k in ("x", "sel", "w", "out", "ws"):
+        assert call(**{k: None}) == B.BMX_ERR_ARG and b"null pointer" in L.bmx_last_error()
+    d = B.MoeDesc(4096, 1536, 288, 8, 0, 0, 1, 0.0, ctypes.c_void_p(16), None, ctypes.c_void_p(32))
+    for T, path in ((1, 0), (9, 0), (300, 0), (3, 4)):
+        need = L.bmx_moe_workspace(ctypes.byref(d), T, path)
+        assert call(T=T, path=path, n=need - 1) == B.BMX_ERR_WORKSPACE and str(need).encode() in L.bmx_last_error()
+    assert call(T=0, x=None, sel=None) == B.BMX_OK

@@ -269,6 +269,30 @@ def test_one_token_given_picks(cuda, picks, shared):
     slots.close()
 
 
+def test_bad_layer_enqueues_nothing(cuda):
+    """bmx_moe_slots_forward with a layer its copy agent does not have: refused before the first launch (the workspace keeps
+    its bytes)."""
+    import bmx
+    H, I, E, topk = 256, 128, 8, 2
+    tab = bmx.ExpertTable.random(H, I, E, (bmx.TF_K3,) * 3, seed=3, device=cuda)
+    slots = bmx.ExpertSlots([tab], E, maxj=E, copies="dma")
+    m = bmx.MoELayer(tab, topk, slots=slots)
+    slots.warm(0, range(E))
+    x = torch.randn((1, H), device=cuda).half()
+    sel = torch.tensor([[1, 2]], dtype=torch.int64, device=cuda)
+    w, out = torch.ones((1, topk), device=cuda).half(), torch.zeros((1, H), device=cuda)
+    L = bmx.lib()
+    ws = torch.full((L.bmx_moe_workspace(m.slot_desc, 1, 0),), 0x5A, dtype=torch.uint8, device=cuda)
+    say("bad layer")
+    for li in (-1, 1, 99):
+        rc = L.bmx_moe_slots_forward(m.slot_desc, slots.agent, li, x.data_ptr(), 1, sel.data_ptr(), w.data_ptr(),
+                                     out.data_ptr(), ws.data_ptr(), ws.numel(), 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == bmx._lib.BMX_ERR_ARG and b"bad layer" in L.bmx_last_error()
+    torch.cuda.synchronize()
+    assert bool((ws == 0x5A).all())
+    slots.close()
+
+
 @pytest.mark.parametrize("copies", ["kernel", "dma"])
 def test_prefetch_keeps_outputs(cuda, copies):
     """A decode loop over a stack of layers with homes in pinned host memory, each layer's step followed by a prefetch
