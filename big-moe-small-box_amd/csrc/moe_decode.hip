@@ -528,6 +528,7 @@ constexpr long EP_SMALL = 16384;              // launches with fewer units use U
 // The gate / up epilogue's own line: a wave per unit costs four times the activations of 16 lanes per unit, which shows once
 // the units fill the SIMDs (11,088 units, four splits: 16.8 us against 14.4)
 constexpr long EP_SMALL_GU = 4096;
+static bool gu_grouped(long units) { return units < EP_SMALL_GU; }
 
 // gate / up epilogue: sum of the splits in split order -> fp16 gate / up (the stored GEMV / GEMM results) -> H128 * R * svh
 // -> activation -> * down suh -> H128 * R -> fp16 down-input row (exllamav3 kernel A epilogue order,
@@ -985,8 +986,8 @@ int launch_epilogue(const GvArgs& a, int stage, hipStream_t s)
     switch (stage)
     {
         case BMX_STAGE_ACT:
-            if (gu >= EP_SMALL_GU) hipLaunchKernelGGL(k_gu_epi<4>, wgs(gu, 4), dim3(GV_THREADS), 0, s, a);
-            else hipLaunchKernelGGL(k_gu_epi_w, wgs(gu, 1), dim3(GV_THREADS), 0, s, a);
+            if (gu_grouped(gu)) hipLaunchKernelGGL(k_gu_epi_w, wgs(gu, 1), dim3(GV_THREADS), 0, s, a);
+            else hipLaunchKernelGGL(k_gu_epi<4>, wgs(gu, 4), dim3(GV_THREADS), 0, s, a);
             break;
         case BMX_STAGE_COMBINE:
             if (cmb >= EP_SMALL) hipLaunchKernelGGL(k_dn_combine, wgs(cmb, 4), dim3(GV_THREADS), 0, s, a);
@@ -1004,7 +1005,7 @@ int launch_epilogue(const GvArgs& a, int stage, hipStream_t s)
 int decode_gu_grouped(const MoeShape& m)
 {
     const DecodePlan p = decode_plan(m);
-    return (long)p.R_max * p.NB < EP_SMALL_GU ? 1 : 0;     // k_gu_epi_w and the one-token down prologue: gu_epi_wave
+    return gu_grouped((long)p.R_max * p.NB) ? 1 : 0;       // k_gu_epi_w and the one-token down prologue: gu_epi_wave
 }
 
 // ---- plan ------------------------------------------------------------------------------------------------------------
@@ -1210,11 +1211,12 @@ int launch_decode_experts(const MoeShape& m, const void* x, const bmx_routes* r,
     // for: the down GEMV computes the activation of its k-range itself, once per output block instead of once, for
     // one launch and one round trip through memory fewer. Worth it while the down workgroups start in one round (5 per
     // compute unit), so the repeated epilogues run side by side: 9 experts of H 4096, I 1536 (1,152 workgroups) 46.7 ->
-    // 44.8 us; in two rounds (7 experts of H 5120, I 2304: 1,680) it costs 64.8 -> 66.5.
+    // 44.8 us; in two rounds (7 experts of H 5120, I 2304: 1,680) it costs 64.8 -> 66.5. Only where the separate epilogue
+    // would add the k-splits in the same order (decode_gu_grouped), so that both forms and the exact CPU lane agree.
     a.gu_half = 0;
     a.act_in_down = rows_per_group_of(m.T) == 1 && (stages & (1 << BMX_STAGE_ACT)) && (stages & (1 << BMX_STAGE_DOWN)) &&
                     !act_rows && (m.H / 128 <= 16 || (long)p.G_max * p.NBH * p.KS_dn <= 5L * cu_count()) &&
-                    act_in_down_allowed();
+                    gu_grouped((long)p.R_max * p.NB) && act_in_down_allowed();
     switch (rows_per_group_of(m.T))
     {
         case 1: launch_mr<1>(a, q, stages, s, rf, pf); break;

@@ -170,6 +170,32 @@ def test_cpu_lane_rows_bitexact_sequential_splits(cuda):
         say("expert", e, "rows bit-identical", r1 - r0)
 
 
+@pytest.mark.parametrize("I,grouped", [(16256, 1), (16384, 0)])
+def test_one_token_both_sides_of_the_epilogue_line(cuda, monkeypatch, I, grouped):
+    """One token of 32 picks, 4,064 and 4,096 units of the gate / up epilogue (below and at the line where it stops adding
+    the k-splits in four groups), eight splits: the down GEMV's own activation, the separate epilogue (BMX_ACT_IN_DOWN=0)
+    and the CPU lane at the reported order give the same bits."""
+    import bmx
+    from bmx import cpu_lane
+    H, E = 1024, 32
+    monkeypatch.setenv("BMX_KS_GU", "8")
+    tab = bmx.ExpertTable.random(H, I, E, (bmx.TF_K2, bmx.TF_K3, bmx.TF_K2), seed=17, device=cuda)
+    x = torch.randn((1, H), generator=torch.Generator(device=cuda).manual_seed(18), device=cuda).half()
+    sel = torch.arange(E, dtype=torch.int64, device=cuda).view(1, E)
+    desc = tab.desc(E)
+    routes = bmx.ops.dispatch(sel, E, 0, False, 1)
+    say("epilogue line", I)
+    y, _ = bmx.ops.moe_experts(desc, x, routes, path=bmx.PATH_DECODE)
+    monkeypatch.setenv("BMX_ACT_IN_DOWN", "0")
+    ref, _ = bmx.ops.moe_experts(desc, x, routes, path=bmx.PATH_DECODE)
+    torch.cuda.synchronize()
+    assert cpu_lane.decode_splits(desc, 1)[0] == 8 and cpu_lane.decode_splits(desc, 1)[2] == grouped
+    assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
+    for e in (0, 31):
+        yc = cpu_lane.expert_rows(tab.host_expert(e), H, I, x.cpu().numpy(), *cpu_lane.decode_splits(desc, 1), threads=16)
+        assert (yc.view(np.uint32) == y[e:e + 1].cpu().numpy().view(np.uint32)).all(), e
+
+
 def test_cpu_lane_time_c2_expert(cuda):
     """Reported, not asserted: one C2-shaped expert (H 4096, I 1536, K 3) for one token on the host's cores, the exact
     lane once, the fast mode warm (one expert again and again) and cold (32 experts in turn, 227 MB)."""
