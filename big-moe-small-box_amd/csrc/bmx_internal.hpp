@@ -61,7 +61,11 @@ struct DecodePlan {
     int KS_gu, KS_dn, NB, NBH, G_max, R_max;
     size_t part_gu_bytes, part_dn_bytes, counters;
 };
-DecodePlan decode_plan(const MoeShape& m);
+// The rules that take more k-splits than fill the chip at first (several-token GEMV calls; mid-size calls of few rows or few
+// waves) cost workspace. They apply while the call's partial sums and rows stay within this, so that no call outgrows
+// bmx_moe_layer_scratch by them; extra = false is the plan without them.
+constexpr size_t EXTRA_SPLITS_WS = BMX_SCRATCH_BYTES / 4 * 3;
+DecodePlan decode_plan(const MoeShape& m, bool extra = true);
 int decode_gu_grouped(const MoeShape& m);     // 1: the gate / up epilogue sums the k-splits in four interleaved groups
 size_t decode_ws_bytes(const MoeShape& m);
 // ws layout: [part_gu][part_dn][act rows (used when act_rows == NULL)]; stages: 1 = gate/up, 2 = down (+ combine)

@@ -1043,7 +1043,12 @@ static long target_wgs()
     return (v && *v) ? atol(v) : 1024;
 }
 
-DecodePlan decode_plan(const MoeShape& m)
+static size_t decode_plan_bytes(const DecodePlan& p, int I)
+{
+    return align_up(p.part_gu_bytes, 256) + align_up(p.part_dn_bytes, 256) + align_up((size_t)p.R_max * I * 2, 256);
+}
+
+DecodePlan decode_plan(const MoeShape& m, bool extra)
 {
     DecodePlan p;
     const int MR = rows_per_group_of(m.T);
@@ -1055,33 +1060,35 @@ DecodePlan decode_plan(const MoeShape& m)
     const long uniq = n < ne ? n : ne;
     const long est = uniq + (long)(m.T > MR ? (m.T * m.topk) / (MR * 4) : 0);
     // the staged input rows (NM matrices x MR rows x k-range fp16) must fit GV_LDS_X
+    auto fit = [](int k, int ks, int max_kr) {
+        while (k / ks > max_kr) { int d = ks + 1; while ((k / 128) % d) ++d; ks = d; }
+        return ks;
+    };
     const int max_kr_gu = GV_LDS_X / (2 * MR * 2), max_kr_dn = GV_LDS_X / (MR * 2);
-    int ks = pick_split(m.H / 128, est * p.NB, target_wgs(), "BMX_KS_GU");
-    if (MR > 1)
+    auto set_gu = [&](int ks) {
+        p.KS_gu = ks;
+        p.part_gu_bytes = (size_t)ks * p.R_max * p.NB * 256 * 4;
+    };
+    p.KS_dn = fit(m.I, pick_split(m.I / 128, est * p.NBH, target_wgs(), "BMX_KS_DN"), max_kr_dn);
+    p.part_dn_bytes = (size_t)p.KS_dn * p.R_max * p.NBH * 128 * 4;
+    p.counters = 0;
+    const int ks = fit(m.H, pick_split(m.H / 128, est * p.NB, target_wgs(), "BMX_KS_GU"), max_kr_gu);
+    set_gu(ks);
+    if (extra && MR > 1)
     {
         // several tokens: four workgroups start per compute unit, so just over 1,024 of them run as two rounds, the second
         // nearly empty; twice the target unless a split would get under 256 of k (its rotation and start then cost more: 4
         // tokens of H 2048 46.4 -> 47.6 us). H 4096, 9 experts a token: 2 tokens 75.3 -> 73.8, 3 tokens 107 -> 98.5, 4 tokens
-        // 124.9 -> 121.0; with 6 experts and I 2048, 4 tokens 103.1 -> 99.3
+        // 124.9 -> 121.0; with 6 experts and I 2048, 4 tokens 103.1 -> 99.3. A prime factor of H / 128 can make it many more
+        // splits (H 5888: 2 -> 23 at the same time, 227 us), so the call's workspace is looked at.
         const int k2 = pick_split(m.H / 128, est * p.NB, 2 * target_wgs(), "BMX_KS_GU");
-        if (m.H / k2 >= 256) ks = k2;
+        if (m.H / k2 >= 256) set_gu(fit(m.H, k2, max_kr_gu));
+        if (decode_plan_bytes(p, m.I) > EXTRA_SPLITS_WS) set_gu(ks);
     }
-    while (m.H / ks > max_kr_gu) { int d = ks + 1; while ((m.H / 128) % d) ++d; ks = d; }
-    p.KS_gu = ks;
-    ks = pick_split(m.I / 128, est * p.NBH, target_wgs(), "BMX_KS_DN");
-    while (m.I / ks > max_kr_dn) { int d = ks + 1; while ((m.I / 128) % d) ++d; ks = d; }
-    p.KS_dn = ks;
-    p.part_gu_bytes = (size_t)p.KS_gu * p.R_max * p.NB * 256 * 4;
-    p.part_dn_bytes = (size_t)p.KS_dn * p.R_max * p.NBH * 128 * 4;
-    p.counters = 0;
     return p;
 }
 
-size_t decode_ws_bytes(const MoeShape& m)
-{
-    const DecodePlan p = decode_plan(m);
-    return align_up(p.part_gu_bytes, 256) + align_up(p.part_dn_bytes, 256) + align_up((size_t)p.R_max * m.I * 2, 256);
-}
+size_t decode_ws_bytes(const MoeShape& m) { return decode_plan_bytes(decode_plan(m), m.I); }
 
 // stages: bit i = BMX_STAGE i (GATE_UP, ACT, DOWN, COMBINE, DOWN_OUT; PREP launches nothing here: the GEMV rotates)
 // the routing gate / up GEMV for ceil(E / 64) = J
@@ -1254,15 +1261,35 @@ static int split_ratio2()
     return q < 0 ? 0 : q;
 }
 
+// Both kernels' plans over one partial layout; the plans without extra splits when the larger of each outgrow the limit
+// together.
+struct SplitPlan {
+    DecodePlan p;
+    int ks_gu_mid, ks_dn_mid;
+    size_t part_gu, part_dn, act, xt;
+};
+
+static SplitPlan split_plan(const MoeShape& m)
+{
+    SplitPlan q;
+    for (bool extra : {true, false})
+    {
+        q.p = decode_plan(m, extra);
+        split_mid_splits(m, &q.ks_gu_mid, &q.ks_dn_mid, extra);
+        const size_t R = (size_t)q.p.R_max;
+        q.part_gu = align_up((size_t)std::max(q.p.KS_gu, q.ks_gu_mid) * R * q.p.NB * 256 * 4, 256);
+        q.part_dn = align_up((size_t)std::max(q.p.KS_dn, q.ks_dn_mid) * R * q.p.NBH * 128 * 4, 256);
+        q.act = align_up(R * m.I * 2, 256);
+        q.xt = align_up((size_t)2 * R * m.H * 2, 256);
+        if (q.part_gu + q.part_dn + q.act + q.xt <= EXTRA_SPLITS_WS) break;
+    }
+    return q;
+}
+
 size_t split_ws_bytes(const MoeShape& m)
 {
-    const DecodePlan p = decode_plan(m);
-    int ksg = 1, ksd = 1;
-    split_mid_splits(m, &ksg, &ksd);
-    const size_t R = (size_t)p.R_max;
-    return align_up((size_t)std::max(p.KS_gu, ksg) * R * p.NB * 256 * 4, 256) +
-           align_up((size_t)std::max(p.KS_dn, ksd) * R * p.NBH * 128 * 4, 256) + align_up(R * m.I * 2, 256) +
-           align_up((size_t)2 * R * m.H * 2, 256);
+    const SplitPlan q = split_plan(m);
+    return q.part_gu + q.part_dn + q.act + q.xt;
 }
 
 // One call over both kernels: the heavy experts' rows (split_heavy) on k_mid_gemm over (expert, 32-row chunk)
@@ -1278,10 +1305,8 @@ int launch_split_experts(const MoeShape& m, const void* x, const bmx_routes* r, 
         return set_error(BMX_ERR_WORKSPACE, "moe experts: workspace %zu < %zu", ws_bytes, split_ws_bytes(m));
     if (!r->row_expert || !r->counts || !r->uexp || !r->nuniq)
         return set_error(BMX_ERR_ARG, "moe experts: split path needs the routes' counts, uexp, nuniq and row_expert");
-    const DecodePlan p = decode_plan(m);
-    int ksg = 1, ksd = 1;
-    split_mid_splits(m, &ksg, &ksd);
-    const size_t R = (size_t)p.R_max;
+    const SplitPlan q = split_plan(m);
+    const DecodePlan& p = q.p;
     char* w = static_cast<char*>(ws);
     GvArgs a;
     a.experts = m.experts; a.shared = m.shared_ex; a.E = m.E; a.H = m.H; a.I = m.I; a.act = m.act; a.gated = m.gated;
@@ -1289,12 +1314,12 @@ int launch_split_experts(const MoeShape& m, const void* x, const bmx_routes* r, 
     a.x = static_cast<const uint16_t*>(x);
     a.row_token = r->row_token; a.groups = r->groups; a.ngroups = r->ngroups; a.row_expert = r->row_expert;
     a.part_gu = reinterpret_cast<float*>(w);
-    w += align_up((size_t)std::max(p.KS_gu, ksg) * R * p.NB * 256 * 4, 256);
+    w += q.part_gu;
     a.part_dn = reinterpret_cast<float*>(w);
-    w += align_up((size_t)std::max(p.KS_dn, ksd) * R * p.NBH * 128 * 4, 256);
+    w += q.part_dn;
     uint16_t* own_act = reinterpret_cast<uint16_t*>(w);
     a.act_rows = act_rows ? static_cast<uint16_t*>(act_rows) : own_act;
-    w += align_up(R * m.I * 2, 256);
+    w += q.act;
     a.xt = reinterpret_cast<uint16_t*>(w);
     a.y_rows = y_rows;
     a.KS_gu = p.KS_gu; a.KS_dn = p.KS_dn; a.NB = p.NB; a.NBH = p.NBH; a.R_max = p.R_max;
@@ -1309,12 +1334,12 @@ int launch_split_experts(const MoeShape& m, const void* x, const bmx_routes* r, 
     a.split_min = split_min_rows();
     a.split_ratio2 = split_ratio2() > 0 ? split_ratio2() : 1 << 30;
     a.split_chunks = (m.T + 31) / 32;          // an expert has at most one row per token
-    a.KS_gu_mid = ksg;
-    a.KS_dn_mid = ksd;
+    a.KS_gu_mid = q.ks_gu_mid;
+    a.KS_dn_mid = q.ks_dn_mid;
     a.counts = r->counts; a.uexp = r->uexp; a.nuniq = r->nuniq;
     GvArgs b = a;                              // the mid-size kernel's view: its own k-splits
-    b.KS_gu = ksg;
-    b.KS_dn = ksd;
+    b.KS_gu = q.ks_gu_mid;
+    b.KS_dn = q.ks_dn_mid;
     const int nu_max = (int)std::min<long>((long)m.T * m.topk, m.E) + (m.shared ? 1 : 0);
     const int MR = rows_per_group_of(m.T);
     auto gemv = [&](int st) {

@@ -211,7 +211,7 @@ int launch_epilogue(const GvArgs& a, int stage, hipStream_t s);
 // split path, moe_prefill.hip: the k-splits of the mid-size kernel for a call, and the launch of the heavy experts' prep
 // (BMX_STAGE_PREP), gate / up GEMMs (any gate / up stage, with a.filter) or down GEMMs (BMX_STAGE_DOWN); a carries
 // the mid-size splits in KS_gu / KS_dn
-void split_mid_splits(const MoeShape& m, int* ks_gu, int* ks_dn);
+void split_mid_splits(const MoeShape& m, int* ks_gu, int* ks_dn, bool extra);
 void launch_split_mid(const GvArgs& a, int stage, int nu_max, hipStream_t s);
 
 }  // namespace bmx

@@ -634,33 +634,44 @@ struct MidPlan {
 // steps, above them 16. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60 experts of H 4096,
 // I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I 2048) 8 x 4: 86, 4 x 4:
 // 92, 16 x 4: 95, 16 x 16: 103; 77 tokens (693 rows, ~150 experts) 16 x 16: 547, 16 x 8: 560, 16 x 32: 549, 32 x 16: 561, 8 x 8: 608.
-// A matrix's partials past MID_FEW_BYTES keep the 16 steps, so no call outgrows bmx_moe_layer_scratch by them.
+// A matrix's partials past MID_FEW_BYTES keep the 16 steps, and so does a call past EXTRA_SPLITS_WS.
 constexpr int MID_FEW_ROWS = 160;
 constexpr size_t MID_FEW_BYTES = 12u << 20;
-static int mid_split(int ksteps, bool down, int rows, size_t split_bytes)
+static int mid_split(int ksteps, bool down, int rows, size_t split_bytes, bool extra)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
     const int min_steps = (v && *v) ? atoi(v) : 16, few_steps = down ? 4 : 8;
-    const bool few = !(v && *v) && rows <= MID_FEW_ROWS;
+    const bool few = extra && !(v && *v) && rows <= MID_FEW_ROWS;
     for (int d = ksteps; d > 1; --d)
         if (ksteps % d == 0 && (ksteps / d >= min_steps || (few && ksteps / d >= few_steps && d * split_bytes <= MID_FEW_BYTES)))
             return d;
     return 1;
 }
 
-static MidPlan mid_plan(const MoeShape& m)
+static size_t mid_plan_bytes(const MidPlan& p)
+{
+    return align_up(p.xt_bytes, 256) + align_up(p.part_gu_bytes, 256) + align_up(p.act_bytes, 256) +
+           align_up(p.part_dn_bytes, 256);
+}
+
+static MidPlan mid_plan(const MoeShape& m, bool extra = true)
 {
     MidPlan p;
     p.NB = m.I / 128;
     p.NBH = m.H / 128;
     p.G_max = groups_max(m.T, m.topk, m.E, m.shared, MID_M);
     p.R_max = m.T * m.topk + (m.shared ? m.T : 0);
-    p.KS_gu = mid_split(m.H / 64, false, p.R_max, (size_t)p.R_max * p.NB * 1024);
-    p.KS_dn = mid_split(m.I / 64, true, p.R_max, (size_t)p.R_max * p.NBH * 512);
     p.xt_bytes = (size_t)2 * p.R_max * m.H * 2;
-    p.part_gu_bytes = (size_t)p.KS_gu * p.R_max * p.NB * 256 * 4;
     p.act_bytes = (size_t)p.R_max * m.I * 2;
-    p.part_dn_bytes = (size_t)p.KS_dn * p.R_max * p.NBH * 128 * 4;
+    const size_t gu = (size_t)p.R_max * p.NB * 256 * 4, dn = (size_t)p.R_max * p.NBH * 128 * 4;     // one split's partials
+    for (bool ex : {extra, false})
+    {
+        p.KS_gu = mid_split(m.H / 64, false, p.R_max, gu, ex);
+        p.KS_dn = mid_split(m.I / 64, true, p.R_max, dn, ex);
+        p.part_gu_bytes = p.KS_gu * gu;
+        p.part_dn_bytes = p.KS_dn * dn;
+        if (mid_plan_bytes(p) <= EXTRA_SPLITS_WS) break;
+    }
     return p;
 }
 
@@ -669,12 +680,7 @@ int mid_rows_per_group() { return MID_M; }
 // workgroups across a matrix's 128-column blocks
 static int mid_blocks(int nb128) { return (nb128 + MID_WAVES - 1) / MID_WAVES; }
 
-size_t mid_ws_bytes(const MoeShape& m)
-{
-    const MidPlan p = mid_plan(m);
-    return align_up(p.xt_bytes, 256) + align_up(p.part_gu_bytes, 256) + align_up(p.act_bytes, 256) +
-           align_up(p.part_dn_bytes, 256);
-}
+size_t mid_ws_bytes(const MoeShape& m) { return mid_plan_bytes(mid_plan(m)); }
 
 int launch_mid_experts(const MoeShape& m, const void* x, const bmx_routes* r, float* y_rows, void* act_rows, void* ws,
                        size_t ws_bytes, float* combine_out, const void* combine_w, hipStream_t s, int stages)
@@ -737,9 +743,9 @@ int launch_mid_experts(const MoeShape& m, const void* x, const bmx_routes* r, fl
 }
 
 // ---- split path: the heavy experts' share ---------------------------------------------------------------------------
-void split_mid_splits(const MoeShape& m, int* ks_gu, int* ks_dn)
+void split_mid_splits(const MoeShape& m, int* ks_gu, int* ks_dn, bool extra)
 {
-    const MidPlan p = mid_plan(m);
+    const MidPlan p = mid_plan(m, extra);
     *ks_gu = p.KS_gu;
     *ks_dn = p.KS_dn;
 }

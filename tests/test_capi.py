@@ -159,3 +159,26 @@ def test_moe_slots_forward_checks():
         need = L.bmx_moe_workspace(ctypes.byref(d), T, path)
         assert call(T=T, path=path, n=need - 1) == B.BMX_ERR_WORKSPACE and str(need).encode() in L.bmx_last_error()
     assert call(T=0, x=None, sel=None) == B.BMX_OK
+
+
+@pytest.mark.parametrize("H,I,E,topk,shared,T,path", [
+    (4096, 5888, 8, 2, 1, 32, 1), (11520, 1408, 8, 2, 1, 32, 1), (1792, 11008, 8, 2, 1, 32, 1),
+    (14464, 2048, 512, 32, 1, 1, 4), (5504, 2816, 512, 32, 0, 2, 4), (12416, 768, 512, 32, 0, 3, 4),
+    (1408, 4096, 512, 32, 0, 5, 4), (8576, 2304, 384, 6, 1, 7, 4), (13184, 3072, 8, 2, 1, 8, 4),
+    (1664, 8192, 64, 8, 1, 8, 4), (1408, 14336, 8, 2, 1, 16, 4), (12032, 2304, 8, 2, 0, 32, 4)])
+def test_extra_splits_stay_in_the_scratch_array(H, I, E, topk, shared, T, path):
+    """Calls whose plan with the fewest k-splits that fill the chip needs 49 to 64 MB: the rules that take more splits leave
+    them within bmx_moe_layer_scratch."""
+    import bmx
+    B = bmx._lib
+    d = B.MoeDesc(H, I, E, topk, 0, 0, 1, 0.0, ctypes.c_void_p(16), ctypes.c_void_p(32) if shared else None)
+    assert 0 < bmx.lib().bmx_moe_layer_workspace(ctypes.byref(d), T, path) <= 64 << 20
+
+
+def test_extra_splits_taken():
+    """The same rules where they pay: a 3-token call of H 4096, I 1536 takes 8 gate / up splits, not 4."""
+    import bmx
+    B = bmx._lib
+    d = B.MoeDesc(4096, 1536, 288, 8, 0, 0, 1, 0.0, ctypes.c_void_p(16), ctypes.c_void_p(32))
+    v = [ctypes.c_int() for _ in range(3)]
+    assert bmx.lib().bmx_decode_splits(ctypes.byref(d), 3, *map(ctypes.byref, v)) == 0 and v[0].value == 8
