@@ -628,24 +628,40 @@ struct MidPlan {
     size_t xt_bytes, part_gu_bytes, act_bytes, part_dn_bytes;
 };
 
-// k-split: the most splits that keep at least min_steps k-steps of 64 each, gate / up (BMX_MID_MIN_STEPS) and down
-// (BMX_MID_MIN_STEPS_DN). Splits even out the SIMDs' shares (the routing, unknown here, may put all rows on a few experts),
-// at the price of partial sums that the epilogues add. Up to MID_FEW_ROWS dispatch rows the partials are small: 8 and 4
-// steps, above them 16. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60 experts of H 4096,
-// I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I 2048) 8 x 4: 86, 4 x 4:
-// 92, 16 x 4: 95, 16 x 16: 103; 77 tokens (693 rows, ~150 experts) 16 x 16: 547, 16 x 8: 560, 16 x 32: 549, 32 x 16: 561, 8 x 8: 608.
-// A matrix's partials past MID_FEW_BYTES keep the 16 steps, and so does a call past EXTRA_SPLITS_WS.
+// k-split: the most splits that keep at least 16 k-steps of 64 each, gate / up and down (BMX_MID_MIN_STEPS,
+// BMX_MID_MIN_STEPS_DN: that many instead, and none of the rules below). More splits even out the SIMDs' shares and fill a
+// chip that the call's units leave idle, at the price of partial sums that the epilogues add. Two rules take them, down to
+// 8 and 4 steps:
+// - Up to MID_FEW_ROWS dispatch rows the partials are small (at most MID_FEW_BYTES a matrix), and the routing, unknown
+//   here, may put all rows on a few experts. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60
+//   experts of H 4096, I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I
+//   2048) 8 x 4: 86, 4 x 4: 92, 16 x 4: 95, 16 x 16: 103. 64 experts of H 2048, I 768, 8 x 4 against 16 x 16: 128 rows 81
+//   against 85, 192 rows 87 against 88, 256 rows 92 against 90, 512 rows 98 against 94; 77 tokens (693 rows, ~150 experts)
+//   16 x 16: 547, 8 x 8: 608.
+// - Above that, splits one after another while a matrix has fewer waves than the chip SIMDs (MID_FILL), counting one group
+//   per expert the picks can reach or per 32 rows: layers of few experts. With 16 x 16 steps and now: 32 experts of H 1024,
+//   I 1024, 192 rows (256 waves a matrix) 79 -> 52 us; 8 of H 2048, I 1024, 192 rows (256 and 128 waves) 110 -> 85; 17 of H
+//   1024, I 512, 1,000 rows 77 -> 63; 8 of H 4096, I 2048, 256 rows (1,024 and 512) 151 -> 147. Past the line they cost
+//   more than they give: 8 of H 4096, I 2048, 800 rows (3,200 and 1,600 waves) 196 at 16 x 16, 218 at 8 x 8; 64 of H 2048,
+//   I 768, 768 rows (1,536 and 1,024) 101 and 108.
+// A call past EXTRA_SPLITS_WS keeps the 16 steps.
 constexpr int MID_FEW_ROWS = 160;
 constexpr size_t MID_FEW_BYTES = 12u << 20;
-static int mid_split(int ksteps, bool down, int rows, size_t split_bytes, bool extra)
+constexpr long MID_FILL = 1024;
+static int mid_split(int ksteps, bool down, int rows, size_t split_bytes, long waves, bool extra)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
     const int min_steps = (v && *v) ? atoi(v) : 16, few_steps = down ? 4 : 8;
-    const bool few = extra && !(v && *v) && rows <= MID_FEW_ROWS;
-    for (int d = ksteps; d > 1; --d)
-        if (ksteps % d == 0 && (ksteps / d >= min_steps || (few && ksteps / d >= few_steps && d * split_bytes <= MID_FEW_BYTES)))
-            return d;
-    return 1;
+    extra = extra && !(v && *v);
+    int best = 1;
+    for (int d = 2; d <= ksteps; ++d)
+    {
+        if (ksteps % d) continue;
+        const bool few = extra && ksteps / d >= few_steps &&
+                         (rows <= MID_FEW_ROWS ? d * split_bytes <= MID_FEW_BYTES : best * waves < MID_FILL);
+        if (ksteps / d >= min_steps || few) best = d;
+    }
+    return best;
 }
 
 static size_t mid_plan_bytes(const MidPlan& p)
@@ -664,10 +680,11 @@ static MidPlan mid_plan(const MoeShape& m, bool extra = true)
     p.xt_bytes = (size_t)2 * p.R_max * m.H * 2;
     p.act_bytes = (size_t)p.R_max * m.I * 2;
     const size_t gu = (size_t)p.R_max * p.NB * 256 * 4, dn = (size_t)p.R_max * p.NBH * 128 * 4;     // one split's partials
+    const long groups = std::max<long>(std::min(m.E, m.T * m.topk) + (m.shared ? 1 : 0), p.R_max / MID_M);
     for (bool ex : {extra, false})
     {
-        p.KS_gu = mid_split(m.H / 64, false, p.R_max, gu, ex);
-        p.KS_dn = mid_split(m.I / 64, true, p.R_max, dn, ex);
+        p.KS_gu = mid_split(m.H / 64, false, p.R_max, gu, 2 * groups * p.NB, ex);
+        p.KS_dn = mid_split(m.I / 64, true, p.R_max, dn, groups * p.NBH, ex);
         p.part_gu_bytes = p.KS_gu * gu;
         p.part_dn_bytes = p.KS_dn * dn;
         if (mid_plan_bytes(p) <= EXTRA_SPLITS_WS) break;

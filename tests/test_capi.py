@@ -182,3 +182,23 @@ def test_extra_splits_taken():
     d = B.MoeDesc(4096, 1536, 288, 8, 0, 0, 1, 0.0, ctypes.c_void_p(16), ctypes.c_void_p(32))
     v = [ctypes.c_int() for _ in range(3)]
     assert bmx.lib().bmx_decode_splits(ctypes.byref(d), 3, *map(ctypes.byref, v)) == 0 and v[0].value == 8
+
+
+@pytest.mark.parametrize("H,I,E,topk,shared,T,ks_gu,ks_dn", [
+    (1024, 1024, 32, 4, 0, 40, 2, 4),      # 160 rows: the rule for few rows
+    (1024, 1024, 32, 4, 0, 48, 2, 4),      # 192 rows, 512 and 256 waves unsplit
+    (1024, 512, 16, 4, 1, 200, 2, 2),      # 1,000 rows: a group per 32 rows
+    (4096, 2048, 8, 2, 0, 128, 4, 4),      # 256 rows, 1,024 waves at 4 gate / up splits: they stay
+    (4096, 2048, 8, 2, 0, 96, 4, 4),       # the same groups
+    (4096, 1920, 8, 2, 0, 96, 8, 5),       # 960 waves at 4: 8; down 512 at 2 -> the next divisors of 30 steps: 3, 5
+    (4096, 2048, 8, 2, 0, 400, 4, 2),      # 800 rows: both matrices full
+    (1024, 1024, 32, 4, 0, 400, 1, 1),     # 1,600 rows: the splits would need more than 48 MiB
+    (4096, 1536, 288, 8, 1, 77, 4, 1)])    # many experts
+def test_mid_splits(H, I, E, topk, shared, T, ks_gu, ks_dn):
+    """k-splits of the mid-size path, from its workspace: rotated rows, gate / up partials, activations, down partials."""
+    import bmx
+    B = bmx._lib
+    d = B.MoeDesc(H, I, E, topk, 0, 0, 1, 0.0, ctypes.c_void_p(16), ctypes.c_void_p(32) if shared else None)
+    R = T * (topk + shared)
+    want = sum((n + 255) // 256 * 256 for n in (4 * R * H, ks_gu * R * I * 8, 2 * R * I, ks_dn * R * H * 4))
+    assert bmx.lib().bmx_experts_workspace(ctypes.byref(d), T, B.PATH_MID) == want
