@@ -638,36 +638,31 @@ struct MidPlan {
 //   2048) 8 x 4: 86, 4 x 4: 92, 16 x 4: 95, 16 x 16: 103. 64 experts of H 2048, I 768, 8 x 4 against 16 x 16: 128 rows 81
 //   against 85, 192 rows 87 against 88, 256 rows 92 against 90, 512 rows 98 against 94; 77 tokens (693 rows, ~150 experts)
 //   16 x 16: 547, 8 x 8: 608.
-// - Above that, splits one after another while a matrix has fewer waves than the chip SIMDs (MID_FILL), counting one group
-//   per expert the picks can reach or per 32 rows: layers of few experts. With 16 x 16 steps and now: 32 experts of H 1024,
-//   I 1024, 192 rows (256 waves a matrix) 79 -> 52 us; 8 of H 2048, I 1024, 192 rows (256 and 128 waves) 110 -> 85; 17 of H
-//   1024, I 512, 1,000 rows 77 -> 63; 8 of H 4096, I 2048, 256 rows (1,024 and 512) 151 -> 147. Past the line they cost
-//   more than they give: 8 of H 4096, I 2048, 800 rows (3,200 and 1,600 waves) 196 at 16 x 16, 218 at 8 x 8; 64 of H 2048,
-//   I 768, 768 rows (1,536 and 1,024) 101 and 108.
-// A call past EXTRA_SPLITS_WS keeps the 16 steps.
+// - Splits one after another while a matrix has fewer waves than the chip SIMDs (MID_FILL), counting one group per expert
+//   the picks can reach or per 32 rows: layers of few experts. With 16 x 16 steps and now: 32 experts of H 1024, I 1024,
+//   192 rows (256 waves a matrix) 79 -> 52 us; 8 of H 2048, I 1024, 192 rows (256 and 128 waves) 110 -> 85; 17 of H 1024,
+//   I 512, 1,000 rows 77 -> 63; 8 of H 4096, I 2048, 256 rows (1,024 and 512) 151 -> 147. Past the line they cost more
+//   than they give: 8 of H 4096, I 2048, 800 rows (3,200 and 1,600 waves) 196 at 16 x 16, 218 at 8 x 8; 64 of H 2048, I
+//   768, 768 rows (1,536 and 1,024) 101 and 108.
+// No split past the 16 steps' that would take the call past EXTRA_SPLITS_WS (gate / up first).
 constexpr int MID_FEW_ROWS = 160;
-constexpr size_t MID_FEW_BYTES = 12u << 20;
+constexpr long MID_FEW_BYTES = 12 << 20;
 constexpr long MID_FILL = 1024;
-static int mid_split(int ksteps, bool down, int rows, size_t split_bytes, long waves, bool extra)
+static int mid_split(int ksteps, bool down, int rows, long split_bytes, long waves, long budget)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
-    const int min_steps = (v && *v) ? atoi(v) : 16, few_steps = down ? 4 : 8;
-    extra = extra && !(v && *v);
+    const bool forced = v && *v;
+    const int min_steps = forced ? atoi(v) : 16, few_steps = down ? 4 : 8;
     int best = 1;
     for (int d = 2; d <= ksteps; ++d)
     {
         if (ksteps % d) continue;
-        const bool few = extra && ksteps / d >= few_steps &&
-                         (rows <= MID_FEW_ROWS ? d * split_bytes <= MID_FEW_BYTES : best * waves < MID_FILL);
+        const long bytes = d * split_bytes;
+        const bool few = !forced && ksteps / d >= few_steps && bytes <= budget &&
+                         ((rows <= MID_FEW_ROWS && bytes <= MID_FEW_BYTES) || best * waves < MID_FILL);
         if (ksteps / d >= min_steps || few) best = d;
     }
     return best;
-}
-
-static size_t mid_plan_bytes(const MidPlan& p)
-{
-    return align_up(p.xt_bytes, 256) + align_up(p.part_gu_bytes, 256) + align_up(p.act_bytes, 256) +
-           align_up(p.part_dn_bytes, 256);
 }
 
 static MidPlan mid_plan(const MoeShape& m, bool extra = true)
@@ -679,16 +674,17 @@ static MidPlan mid_plan(const MoeShape& m, bool extra = true)
     p.R_max = m.T * m.topk + (m.shared ? m.T : 0);
     p.xt_bytes = (size_t)2 * p.R_max * m.H * 2;
     p.act_bytes = (size_t)p.R_max * m.I * 2;
-    const size_t gu = (size_t)p.R_max * p.NB * 256 * 4, dn = (size_t)p.R_max * p.NBH * 128 * 4;     // one split's partials
+    const long gu = (long)p.R_max * p.NB * 256 * 4, dn = (long)p.R_max * p.NBH * 128 * 4;     // one split's partials
     const long groups = std::max<long>(std::min(m.E, m.T * m.topk) + (m.shared ? 1 : 0), p.R_max / MID_M);
-    for (bool ex : {extra, false})
-    {
-        p.KS_gu = mid_split(m.H / 64, false, p.R_max, gu, 2 * groups * p.NB, ex);
-        p.KS_dn = mid_split(m.I / 64, true, p.R_max, dn, groups * p.NBH, ex);
-        p.part_gu_bytes = p.KS_gu * gu;
-        p.part_dn_bytes = p.KS_dn * dn;
-        if (mid_plan_bytes(p) <= EXTRA_SPLITS_WS) break;
-    }
+    auto splits = [&](bool down, long budget) {
+        return down ? mid_split(m.I / 64, true, p.R_max, dn, groups * p.NBH, budget)
+                    : mid_split(m.H / 64, false, p.R_max, gu, 2 * groups * p.NB, budget);
+    };
+    const long room = extra ? (long)EXTRA_SPLITS_WS - (long)(p.xt_bytes + p.act_bytes) : 0;
+    p.KS_gu = splits(false, room - splits(true, 0) * dn);
+    p.KS_dn = splits(true, room - p.KS_gu * gu);
+    p.part_gu_bytes = p.KS_gu * gu;
+    p.part_dn_bytes = p.KS_dn * dn;
     return p;
 }
 
@@ -697,7 +693,12 @@ int mid_rows_per_group() { return MID_M; }
 // workgroups across a matrix's 128-column blocks
 static int mid_blocks(int nb128) { return (nb128 + MID_WAVES - 1) / MID_WAVES; }
 
-size_t mid_ws_bytes(const MoeShape& m) { return mid_plan_bytes(mid_plan(m)); }
+size_t mid_ws_bytes(const MoeShape& m)
+{
+    const MidPlan p = mid_plan(m);
+    return align_up(p.xt_bytes, 256) + align_up(p.part_gu_bytes, 256) + align_up(p.act_bytes, 256) +
+           align_up(p.part_dn_bytes, 256);
+}
 
 int launch_mid_experts(const MoeShape& m, const void* x, const bmx_routes* r, float* y_rows, void* act_rows, void* ws,
                        size_t ws_bytes, float* combine_out, const void* combine_w, hipStream_t s, int stages)

@@ -192,7 +192,10 @@ def test_extra_splits_taken():
     (4096, 2048, 8, 2, 0, 96, 4, 4),       # the same groups
     (4096, 1920, 8, 2, 0, 96, 8, 5),       # 960 waves at 4: 8; down 512 at 2 -> the next divisors of 30 steps: 3, 5
     (4096, 2048, 8, 2, 0, 400, 4, 2),      # 800 rows: both matrices full
-    (1024, 1024, 32, 4, 0, 400, 1, 1),     # 1,600 rows: the splits would need more than 48 MiB
+    (1024, 1024, 32, 4, 0, 400, 2, 2),     # 1,600 rows: four down splits would need more than 48 MiB
+    (4096, 2048, 1, 1, 0, 128, 8, 8),      # one expert's rows: 128, past the few-rows rule's bytes
+    (4096, 2048, 1, 1, 0, 200, 8, 4),      # 6 groups; eight down splits would need more than 48 MiB
+    (4096, 2048, 1, 1, 0, 300, 4, 4),      # 9 groups
     (4096, 1536, 288, 8, 1, 77, 4, 1)])    # many experts
 def test_mid_splits(H, I, E, topk, shared, T, ks_gu, ks_dn):
     """k-splits of the mid-size path, from its workspace: rotated rows, gate / up partials, activations, down partials."""
