@@ -200,10 +200,12 @@ class MoELayer:
             raise ValueError("run_single_expert: y must be fp32 [n, H]")
         if n == 0:
             return y
-        sel = torch.full((n, 1), int(e) + self.routing_first, dtype=torch.int64, device=x.device)
-        desc = self.table.desc(1, self.routing_first, self.act, self.gated, self.act_limit)
-        desc.shared = None
-        routes = ops.dispatch(sel, E, self.routing_first, False, L.lib().bmx_rows_per_group(n, 1, path))
+        # a layer of that one expert: the plans then know that every row is its
+        sel = torch.zeros((n, 1), dtype=torch.int64, device=x.device)
+        desc = self.table.desc(1, 0, self.act, self.gated, self.act_limit)
+        desc.experts += int(e) * ctypes.sizeof(L.Expert)
+        desc.E, desc.shared = 1, None
+        routes = ops.dispatch(sel, 1, 0, False, L.lib().bmx_rows_per_group(n, 1, path))
         rows, _ = ops.moe_experts(desc, x, routes, path)
         y.copy_(rows[:n])            # one expert: its rows are the tokens in order
         return y

@@ -1,4 +1,5 @@
 """Layer calls refuse host tensors before anything is enqueued, and a refused call leaves the layer as it was (CPU only)."""
+import ctypes
 import types
 
 import pytest
@@ -59,3 +60,21 @@ def test_slot_call_refuses_other_shapes(xs, ss, ws):
     x, sel, w = Dev(xs, torch.float16), Dev(ss, torch.int64), Dev(ws, torch.float16)
     with pytest.raises(ValueError, match="of one T"):
         bmx.ops.moe_slots_forward(bare_layer().slot_desc, None, 0, x, sel, w)
+
+
+def test_single_expert_is_a_layer_of_one(monkeypatch):
+    """run_single_expert(e) calls the library for a layer of that expert alone (its record, one expert, no shared one), so
+    the plans count on all rows being its."""
+    import bmx
+    m = bare_layer()
+    got = {}
+    m.act, m.gated, m.act_limit = 0, True, 0.0
+    m.table.desc = lambda topk, first, *a: bmx._lib.MoeDesc(256, 128, 8, topk, first, 0, 1, 0.0, 4096, 8192, None)
+    monkeypatch.setattr(bmx.ops, "dispatch", lambda sel, E, first, shared, rpg: got.update(sel=sel, E=E, first=first, shared=shared))
+    monkeypatch.setattr(bmx.ops, "moe_experts", lambda desc, x, r, path: (got.update(desc=desc), (torch.full((3, 256), 7.0), None))[1])
+    m.routing_first = 100
+    y = m.run_single_expert(torch.zeros((3, 256)), 5, torch.zeros((3, 256)).half())
+    d = got["desc"]
+    assert (d.E, d.topk, d.first, d.shared, d.experts) == (1, 1, 0, None, 4096 + 5 * ctypes.sizeof(bmx._lib.Expert))
+    assert got["E"] == 1 and got["first"] == 0 and not got["shared"] and got["sel"].tolist() == [[0]] * 3
+    assert bool((y == 7.0).all())
