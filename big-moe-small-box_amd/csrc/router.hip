@@ -322,8 +322,13 @@ __global__ __launch_bounds__(RL_WAVES * 64, 2) void k_router_logits_few(const ui
 // 128 bytes of a row per eight lanes and shared through LDS (16-byte chunk c of row r at c ^ (r % 8): eight rows' chunks
 // of one step spread over all banks); the loads run D stages ahead in registers, about 128 KB per workgroup. Operands
 // straight from memory in 32 x 32 tiles, as this kernel once did, touch 32 cache lines per load for a quarter of each
-// and read twice as much. The tile is the largest that still gives most CUs a workgroup. It is bound by the tiles' reads:
-// 2,048 tokens, 384 experts, H 4096: 53.2 -> 20.6 us; 77 tokens, 288 experts: 19.8 -> 10.6.
+// and read twice as much. It is bound by the tiles' reads:
+// 2,048 tokens, 384 experts, H 4096: 53.2 -> 20.6 us; 77 tokens, 288 experts: 19.8 -> 10.6. Larger tiles read less but
+// leave more CUs idle; the lines are where the next size starts its second round on the 256 CUs (us at H 4096):
+//   64 x 64 from 96 tiles: 96 of them (384 experts) 17.6, 32 x 32 17.3; 144: 18.7 and 24.9; 70 (288 experts): 17.3 and 14.2.
+//   32 x 32 from 128 tiles: 144 of them 9.6, 32 x 16 12.8; 120: 9.5 and 9.6; 108 (288 experts): 10.9 and 9.5.
+//   Up to 32 experts 32 x 32 always: a wider tile reads no less of z and its other columns are copies (8,192 tokens, 8
+//   experts: 13.4, 64 x 64 17.7).
 // Workgroups go to the 8 XCDs round-robin: with large tiles (at least 96 of them) the blocks of a token tile are renumbered
 // onto one XCD, whose L2 then reads the tokens once (W, the smaller matrix, is read by all).
 template <int NT, int ER, int D>
@@ -418,7 +423,7 @@ int launch_router_logits(const void* z, const void* W, int T, int H, int E, void
     if (T <= 32 && few <= RL_FEW_LDS)
         hipLaunchKernelGGL(k_router_logits_few, dim3((unsigned)((E + RL_FEW_EB - 1) / RL_FEW_EB)), block,
                            std::max(few, (size_t)RL_WAVES * 4096), s, zp, wp, T, H, E, lp);
-    else if (tiles(64, 64) >= 96)
+    else if (E > 32 && tiles(64, 64) >= 96)
         hipLaunchKernelGGL((k_router_logits<2, 64, 2>), dim3((unsigned)(8 * tiles(512, 64))), block, 0, s, zp, wp, T, H, E, lp);
     else if (tiles(32, 32) >= 128)
         hipLaunchKernelGGL((k_router_logits<1, 32, 4>), dim3((unsigned)tiles(32, 32)), block, 0, s, zp, wp, T, H, E, lp);

@@ -58,6 +58,8 @@ def test_router_logits_projection(cuda, oracle, T, E, H):
                                    (1023, 321, 64),      # one step per quarter
                                    (511, 256, 1088),     # 128 tiles of 32 x 32
                                    (480, 256, 192),      # just below: 16 experts a tile
+                                   (6113, 32, 192),      # up to 32 experts: 32 x 32 tiles at any count
+                                   (6113, 33, 192),      # one more: 64 x 64
                                    (9, 250, 5184)])      # one row past the kernel of few rows, H past its first trip
 def test_router_logits_same_in_every_tile(cuda, oracle, T, E, H):
     """A token's logits are the same bits whatever tile its call takes: the call against calls of 31, 8 and 3 tokens."""
