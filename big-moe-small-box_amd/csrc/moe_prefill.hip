@@ -632,12 +632,12 @@ struct MidPlan {
 // BMX_MID_MIN_STEPS_DN: that many instead, and none of the rules below). More splits even out the SIMDs' shares and fill a
 // chip that the call's units leave idle, at the price of partial sums that the epilogues add. Two rules take them, down to
 // 8 and 4 steps:
-// - Up to MID_FEW_ROWS dispatch rows the partials are small (at most MID_FEW_BYTES a matrix), and the routing, unknown
-//   here, may put all rows on a few experts. Measured (layer us, gate / up steps x down steps): 8 tokens (72 rows, ~60
-//   experts of H 4096, I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96 rows, I
-//   2048) 8 x 4: 86, 4 x 4: 92, 16 x 4: 95, 16 x 16: 103. 64 experts of H 2048, I 768, 8 x 4 against 16 x 16: 128 rows 81
-//   against 85, 192 rows 87 against 88, 256 rows 92 against 90, 512 rows 98 against 94; 77 tokens (693 rows, ~150 experts)
-//   16 x 16: 547, 8 x 8: 608.
+// - While a matrix's partials stay within MID_FEW_BYTES: the routing, unknown here, may put all rows on a few experts, and
+//   partials of that size cost little where it does not. Measured (layer us, gate / up steps x down steps): 8 tokens (72
+//   rows, ~60 experts of H 4096, I 1536) 8 x 4: 165, 16 x 4: 169, 8 x 16: 178, 32 x 16: 194; 16 tokens on ~12 experts (96
+//   rows, I 2048) 8 x 4: 86, 4 x 4: 92, 16 x 4: 95, 16 x 16: 103. 64 experts of H 2048, I 768, 192 and 512 rows: picks
+//   spread 88 -> 83 and 94 -> 92, tokens of one context 74 -> 54 and 82 -> 69. Past 12 MiB the spread calls pay: 18
+//   tokens of the first layer 354 us within it, 362 at 16 MiB; 1,024 rows of the last 105, at 24 MiB 108.
 // - Splits one after another while a matrix has fewer waves than the chip SIMDs (MID_FILL), counting one group per expert
 //   the picks can reach or per 32 rows: layers of few experts. With 16 x 16 steps and now: 32 experts of H 1024, I 1024,
 //   192 rows (256 waves a matrix) 79 -> 52 us; 8 of H 2048, I 1024, 192 rows (256 and 128 waves) 110 -> 85; 17 of H 1024,
@@ -645,10 +645,9 @@ struct MidPlan {
 //   than they give: 8 of H 4096, I 2048, 800 rows (3,200 and 1,600 waves) 196 at 16 x 16, 218 at 8 x 8; 64 of H 2048, I
 //   768, 768 rows (1,536 and 1,024) 101 and 108.
 // No split past the 16 steps' that would take the call past EXTRA_SPLITS_WS (gate / up first).
-constexpr int MID_FEW_ROWS = 160;
 constexpr long MID_FEW_BYTES = 12 << 20;
 constexpr long MID_FILL = 1024;
-static int mid_split(int ksteps, bool down, int rows, long split_bytes, long waves, long budget)
+static int mid_split(int ksteps, bool down, long split_bytes, long waves, long budget)
 {
     const char* v = getenv(down ? "BMX_MID_MIN_STEPS_DN" : "BMX_MID_MIN_STEPS");
     const bool forced = v && *v;
@@ -659,7 +658,7 @@ static int mid_split(int ksteps, bool down, int rows, long split_bytes, long wav
         if (ksteps % d) continue;
         const long bytes = d * split_bytes;
         const bool few = !forced && ksteps / d >= few_steps && bytes <= budget &&
-                         ((rows <= MID_FEW_ROWS && bytes <= MID_FEW_BYTES) || best * waves < MID_FILL);
+                         (bytes <= MID_FEW_BYTES || best * waves < MID_FILL);
         if (ksteps / d >= min_steps || few) best = d;
     }
     return best;
@@ -677,8 +676,8 @@ static MidPlan mid_plan(const MoeShape& m, bool extra = true)
     const long gu = (long)p.R_max * p.NB * 256 * 4, dn = (long)p.R_max * p.NBH * 128 * 4;     // one split's partials
     const long groups = std::max<long>(std::min(m.E, m.T * m.topk) + (m.shared ? 1 : 0), p.R_max / MID_M);
     auto splits = [&](bool down, long budget) {
-        return down ? mid_split(m.I / 64, true, p.R_max, dn, groups * p.NBH, budget)
-                    : mid_split(m.H / 64, false, p.R_max, gu, 2 * groups * p.NB, budget);
+        return down ? mid_split(m.I / 64, true, dn, groups * p.NBH, budget)
+                    : mid_split(m.H / 64, false, gu, 2 * groups * p.NB, budget);
     };
     const long room = extra ? (long)EXTRA_SPLITS_WS - (long)(p.xt_bytes + p.act_bytes) : 0;
     p.KS_gu = splits(false, room - splits(true, 0) * dn);

@@ -185,7 +185,8 @@ def test_extra_splits_taken():
 
 
 @pytest.mark.parametrize("H,I,E,topk,shared,T,ks_gu,ks_dn", [
-    (1024, 1024, 32, 4, 0, 40, 2, 4),      # 160 rows: the rule for few rows
+    (2048, 768, 64, 8, 0, 64, 4, 3),       # 512 rows: 12 MiB of partials a matrix
+    (2048, 768, 64, 8, 0, 65, 2, 2),       # one token past it: the next fewer splits
     (1024, 1024, 32, 4, 0, 48, 2, 4),      # 192 rows, 512 and 256 waves unsplit
     (1024, 512, 16, 4, 1, 200, 2, 2),      # 1,000 rows: a group per 32 rows
     (4096, 2048, 8, 2, 0, 128, 4, 4),      # 256 rows, 1,024 waves at 4 gate / up splits: they stay
@@ -193,7 +194,7 @@ def test_extra_splits_taken():
     (4096, 1920, 8, 2, 0, 96, 8, 5),       # 960 waves at 4: 8; down 512 at 2 -> the next divisors of 30 steps: 3, 5
     (4096, 2048, 8, 2, 0, 400, 4, 2),      # 800 rows: both matrices full
     (1024, 1024, 32, 4, 0, 400, 2, 2),     # 1,600 rows: four down splits would need more than 48 MiB
-    (4096, 2048, 1, 1, 0, 128, 8, 8),      # one expert's rows: 128, past the few-rows rule's bytes
+    (4096, 2048, 1, 1, 0, 128, 8, 8),      # one expert's 128 rows: 16 MiB a matrix, 512 waves unsplit
     (4096, 2048, 1, 1, 0, 200, 8, 4),      # 6 groups; eight down splits would need more than 48 MiB
     (4096, 2048, 1, 1, 0, 300, 4, 4),      # 9 groups
     (4096, 1536, 288, 8, 1, 77, 4, 1)])    # many experts

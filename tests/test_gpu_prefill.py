@@ -149,7 +149,7 @@ MID_LAYERS = [
     ("c3 shape E24 T40", "c3", 24, 40, None, None, [0, 17, 39]),
     ("c1 T4 K4", "c1", 64, 4, None, None, None),
     ("odd blocks H384 I256", "c2", 8, 24, 384, 256, [0, 11, 23]),
-    # few experts, more than 160 rows: splits while the launch has fewer waves than SIMDs (2 x 4; 1 x 5, odd blocks)
+    # few experts: splits while the launch has fewer waves than SIMDs (2 x 4; 1 x 5, odd blocks)
     ("few experts E32 T48", "c2", 32, 48, 1024, 1024, [0, 23, 47]),
     ("few experts odd blocks E8 T40", "c2", 8, 40, 640, 1280, [0, 39]),
 ]
