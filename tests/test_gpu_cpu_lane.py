@@ -140,13 +140,15 @@ def test_layer_with_cpu_experts_bitexact(cuda):
     assert torch.equal(got, want)
 
 
-def test_cpu_lane_rows_bitexact_sequential_splits(cuda):
-    """A launch large enough that the gate / up epilogue sums the k-splits in sequence (not in four groups): rows of
-    two experts from the lane against the GPU's, bit for bit."""
+@pytest.mark.parametrize("T,order", [(255, 1), (256, 0)])
+def test_cpu_lane_rows_bitexact_sequential_splits(cuda, T, order):
+    """4,080 and 4,096 units of the gate / up epilogue, eight splits: below 4,096 it sums them in four groups, from there in
+    sequence. Rows of both experts from the lane at the reported order against the GPU's, bit for bit; the other order
+    differs."""
     import bmx
     from bmx import cpu_lane
-    H, I, E, topk, T = 256, 4096, 8, 3, 171
-    tab = bmx.ExpertTable.random(H, I, E, [(2, 0, 3), (1, 1, 1)] * 4, seed=11, device=cuda)
+    H, I, E, topk = 1024, 1024, 2, 2
+    tab = bmx.ExpertTable.random(H, I, E, [(2, 0, 3), (1, 1, 1)], seed=11, device=cuda)
     rng = np.random.default_rng(11)
     x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float16)).to(cuda)
     lg = torch.from_numpy(rng.standard_normal((T, E)).astype(np.float16)).to(cuda)
@@ -157,7 +159,7 @@ def test_cpu_lane_rows_bitexact_sequential_splits(cuda):
     torch.cuda.synchronize()
     ks_gu, ks_dn, grouped = cpu_lane.decode_splits(desc, T)
     say("sequential case splits", ks_gu, ks_dn, "grouped", grouped)
-    assert grouped == 0
+    assert grouped == order and ks_gu >= 5
     y = y.cpu().numpy()
     rt = routes.row_token.cpu().numpy()
     offs = routes.offsets.cpu().numpy()
@@ -168,6 +170,8 @@ def test_cpu_lane_rows_bitexact_sequential_splits(cuda):
         yc = cpu_lane.expert_rows(tab.host_expert(e), H, I, xs[rt[r0:r1]], ks_gu, ks_dn, grouped, threads=16)
         assert (yc.view(np.uint32) == y[r0:r1].view(np.uint32)).all(), e
         say("expert", e, "rows bit-identical", r1 - r0)
+        other = cpu_lane.expert_rows(tab.host_expert(e), H, I, xs[rt[r0:r1]], ks_gu, ks_dn, 1 - grouped, threads=16)
+        assert (other.view(np.uint32) != y[r0:r1].view(np.uint32)).any(), e
 
 
 @pytest.mark.parametrize("I,grouped", [(16256, 1), (16384, 0)])

@@ -476,3 +476,33 @@ def test_one_token_act_in_down(cuda, fmts, shared):
     finally:
         os.environ.pop("BMX_ACT_IN_DOWN", None)
     assert np.array_equal(a, b) and np.abs(a).max() > 0
+
+
+@pytest.mark.parametrize("H,I,shared", [(4096, 768, False), (2176, 256, True)])
+def test_one_token_act_in_down_one_round(cuda, monkeypatch, H, I, shared):
+    """Above H 2048 the down GEMV computes the activation while its workgroups (groups x output blocks x splits) start in
+    one round, 5 per compute unit: the same bits just below that line (BMX_CU_COUNT one short of it) and with
+    BMX_ACT_IN_DOWN=0, at one gate / up split count."""
+    import bmx
+    from bmx import cpu_lane
+    E, topk = 8, 2
+    monkeypatch.setenv("BMX_KS_GU", str(H // 128 // 8 if H % 1024 == 0 else 1))
+    tab = bmx.ExpertTable.random(H, I, E, (2, 1, 0), shared=shared, seed=13, device=cuda)
+    g = torch.Generator(device=cuda)
+    g.manual_seed(14)
+    x = torch.randn((1, H), generator=g, device=cuda).half()
+    lg = torch.randn((1, E), generator=g, device=cuda).half()
+    layer = bmx.MoELayer(tab, topk, score=bmx.SCORE_SIGMOID, renorm=True, scale=2.0)
+    ks_dn = cpu_lane.decode_splits(layer.desc, 1)[1]
+    cus = -(-(topk + shared) * (H // 128) * ks_dn // 5)
+    say("act in down, one round", H, I, shared, "CUs", cus)
+    outs = []
+    for env in (dict(BMX_CU_COUNT=str(cus)), dict(BMX_CU_COUNT=str(cus - 1)),
+                dict(BMX_CU_COUNT=str(cus), BMX_ACT_IN_DOWN="0")):
+        with monkeypatch.context() as mp:
+            for k, v in env.items():
+                mp.setenv(k, v)
+            assert cpu_lane.decode_splits(layer.desc, 1)[1] == ks_dn
+            outs.append(layer.forward(x, lg, path=bmx.PATH_DECODE).cpu().numpy())
+    assert np.abs(outs[0]).max() > 0
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])

@@ -199,55 +199,45 @@ def test_mid_experts_rows_and_properties(cuda):
     assert torch.equal(b, a * 2)
 
 
-def forced_picks(T, topk, E, plan, seed):
-    """sel [T, topk]: slot k of token t picks plan[k](t); weights random positive"""
-    sel = np.array([[plan[k](t) for k in range(topk)] for t in range(T)], np.int64)
-    assert all(len(set(r)) == topk for r in sel.tolist())
-    w = (np.random.default_rng(seed).random((T, topk)) + 0.25).astype(np.float16)
-    return sel, w
+EDGE_ROWS = (1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 330)      # rows per expert; groups of 128, row blocks of 32
 
 
-PAIR_CASES = [
-    # name, H, I, fmts, shared, T, topk, E, slot plans: expert 0 takes 330 rows (groups 128 128 74: a pair and a
-    # single), expert 1 260 (128, 128, 4: a pair and a single), expert 2 70; odd block counts (H 384, I 384)
-    ("odd blocks, pair + single, shared", 384, 384, (2, 1, 3), True, 330, 2, 6,
-     (lambda t: 0, lambda t: 1 if t < 260 else 2)),
-    # expert 0: 600 rows (five groups: two pairs and a single), expert 1: 300, the rest spread
-    ("two pairs, K4", 1024, 512, (3, 3, 3), False, 600, 3, 9,
-     (lambda t: 0, lambda t: 1 if t < 300 else 2 + t % 7, lambda t: 3 + t % 6 if t < 300 else 2 + (t + 3) % 7)),
-]
-
-
-@pytest.mark.parametrize("name,H,I,fmts,shared,T,topk,E,plan", PAIR_CASES, ids=[c[0] for c in PAIR_CASES])
-def test_prefill_pairs(cuda, oracle, name, H, I, fmts, shared, T, topk, E, plan):
-    """Consecutive 128-row groups of one expert run as one 256-row x 128-column tile (a pair): the same products as
-    one tile per group (BMX_PF_PAIRS=0) bit for bit, and rows of both halves of a pair and of the single group after it
-    within the oracle's tolerance."""
-    import os
+@pytest.mark.parametrize("H,I,fmts,shared", [(384, 640, (2, 1, 3), False),      # odd block counts of both outputs
+                                             (512, 384, (0, 3, 0), True),        # odd gate / up blocks
+                                             (640, 512, (1, 0, 2), False),       # odd down blocks
+                                             (128, 128, (3, 2, 1), False)])      # one block: half of every unit idle
+def test_prefill_group_edges(cuda, oracle, H, I, fmts, shared):
+    """Every row of experts with 1 .. 330 rows (one to four row blocks, full and partial last blocks, a second and a third
+    group) on the prefill GEMM against the mid-size path's rows, and a row at each group's ends against the oracle. Both
+    paths round gate / up, the activation and the rotated rows to fp16 (2^-11 relative each): a row's relative RMS
+    difference stays below 4 x 2^-11."""
     import bmx
+    E, T = len(EDGE_ROWS), sum(EDGE_ROWS)
     tab = bmx.ExpertTable.random(H, I, E, fmts, shared=shared, seed=31, device=cuda)
-    layer = bmx.MoELayer(tab, topk, score=bmx.SCORE_SIGMOID, renorm=True, scale=1.0)
     g = torch.Generator(device=cuda)
     g.manual_seed(32)
     x = torch.randn((T, H), generator=g, device=cuda).half()
-    sel_np, w_np = forced_picks(T, topk, E, plan, 33)
-    sel, w = torch.from_numpy(sel_np).to(cuda), torch.from_numpy(w_np).to(cuda)
-    say("pairs", name, "run")
-    out = layer.run_bszN(x, sel, w, path=PREFILL).clone()
-    os.environ["BMX_PF_PAIRS"] = "0"
-    try:
-        ref = layer.run_bszN(x, sel, w, path=PREFILL).clone()
-    finally:
-        os.environ.pop("BMX_PF_PAIRS", None)
-    torch.cuda.synchronize()
-    say("pairs", name, "max |pairs - singles|", float((out - ref).abs().max()))
-    assert torch.equal(out, ref) and float(out.abs().max()) > 0
-    rows = [0, 127, 128, 200, 255, 256, T - 1]
-    want = oracle_layer(oracle, tab, x.cpu().numpy(), sel_np, w_np, rows)
-    got = out.cpu().numpy()[rows]
-    err_abs, err_rel = float(np.abs(got - want).max()), rel_rms(got, want)
-    say("pairs", name, "oracle rows", rows, "max_abs", err_abs, "rel_rms", err_rel)
-    assert err_abs < MAX_ABS and err_rel < REL_RMS
+    order = np.random.default_rng(33).permutation(np.repeat(np.arange(E), EDGE_ROWS))
+    sel = torch.from_numpy(order.astype(np.int64).reshape(T, 1)).to(cuda)
+    w = torch.ones((T, 1), device=cuda).half()
+    d = tab.desc(1)
+    say("group edges", H, I, fmts)
+    y = {}
+    for path in (PREFILL, MID):
+        r = bmx.ops.dispatch(sel, E, 0, shared, bmx.lib().bmx_rows_per_group(T, 1, path))
+        y[path], _ = bmx.ops.moe_experts(d, x, r, path=path)
+    n = r.rows()
+    assert n == T * (1 + shared) and r.counts[:E].tolist() == list(EDGE_ROWS)
+    a, b = y[PREFILL][:n].double(), y[MID][:n].double()
+    err = ((a - b).square().mean(1) / b.square().mean(1)).sqrt()
+    say("worst row", float(err.max()), "at", int(err.argmax()))
+    assert float(err.max()) < 4 * 2.0 ** -11
+    offs = r.offsets.cpu().numpy()
+    rt = r.row_token.cpu().numpy()
+    ends = sorted({int(rt[i]) for e in range(E) for i in (offs[e], offs[e + 1] - 1)})
+    out = bmx.MoELayer(tab, 1).run_bszN(x, sel, w, path=PREFILL).cpu().numpy()[ends]
+    want = oracle_layer(oracle, tab, x.cpu().numpy(), sel.cpu().numpy(), w.cpu().numpy(), ends)
+    assert float(np.abs(out - want).max()) < MAX_ABS and rel_rms(out, want) < REL_RMS
 
 
 def test_prefill_wide_topk_dropped_picks(cuda, oracle):
