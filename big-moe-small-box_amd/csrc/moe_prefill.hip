@@ -215,7 +215,7 @@ __device__ __forceinline__ void pf_stage_store(const u32x4 (&st)[NMB], u32x4* __
 }
 
 // One operand slot of a wave: operand (CI, Q) of the words w is decoded into b while the products of the operand before
-// it (bp, columns 1 - CI, rows ap) run, one MFMA per 29 / NMB VALU instructions: the two waves of a SIMD march in step
+// it (bp, columns 1 - CI, rows ap) run, one MFMA per 28 / NMB VALU instructions: the two waves of a SIMD march in step
 // from barrier to barrier, so an MFMA burst and a decode burst would each leave the other unit idle.
 template <int F, int HALF, int CI, int Q, int NMB>
 __device__ __forceinline__ void pf_slot(const typename HalfWords<F, HALF>::Buf& w, u32x4& b, const u32x4& bp,
@@ -491,11 +491,11 @@ __device__ __forceinline__ void mid_run(const PfJob& jb, const uint8_t* mat_base
     };
 #pragma unroll
     for (int d = 0; d < MID_D; ++d) fetch(d, d);
+    static_assert(MID_D == 2, "n is even: a split is whole k-steps of 64");
     for (int i = 0; i < n; i += MID_D)
 #pragma unroll
         for (int d = 0; d < MID_D; ++d)
         {
-            if (i + d >= n) break;
             const uint32_t prev = __builtin_amdgcn_mov_dpp(w[d][NW - 1], 0x93, 0xf, 0xf, false);
             mid_mul<F, 0, 0>(prev, w[d], a[d][0], acc);
             mid_mul<F, 1, 0>(prev, w[d], a[d][0], acc);
