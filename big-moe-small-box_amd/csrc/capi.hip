@@ -113,12 +113,16 @@ static bool route_in_gemv_allowed()
 }
 
 // AUTO below the prefill threshold: the mid-size MFMA path from BMX_MID_MIN_TOKENS tokens (8), the GEMV path below.
-// Measured on MI355X (layer us, GEMV / mid-size): GLM-shaped (H 4096, I 1536) T 4 135 / 146, T 6 196 / 190, T 8 234 /
-// 219, T 16 354 / 316, T 32 533 / 432; DeepSeek-shaped (H 4096, I 2048, Zipf routing) T 6 165 / 168, T 8 201 / 193,
-// T 32 524 / 450; 16 tokens on ~10 experts 180 / 107; the 64-expert H 2048 layer crosses over later (T 8 72 / 83, T 16
-// 98 / 94). Mid-size / prefill (128-row groups): DeepSeek-shaped T 86 (516 rows) 819 / 917, T 256 1426 / 1519, T 512
-// 1911 / 1883, T 2048 3546 / 2627; GLM-shaped T 64 554 / 661, T 128 680 / 771. The split path (BMX_PATH_SPLIT) is never
-// chosen here: the mid-size path alone is faster wherever the split path would send a call to the MFMA kernels.
+// Measured on MI355X (layer us, GEMV / mid-size), picks spread: 288 experts of H 4096, I 1536 T 2 76 / 84, T 4 117 / 112, T 7
+// 188 / 160, T 8 227 / 200, T 32 605 / 507; 384 of H 5120, I 2304 T 3 128 / 129, T 7 265 / 239, T 8 296 / 268; 384 of H
+// 4096, I 2048 T 4 109 / 110, T 7 175 / 167, T 8 196 / 189; 64 of H 2048, I 768 T 4 44 / 55, T 7 57 / 63, T 8 63 / 67, T 10
+// 70 / 69. Tokens of one context (about 9 experts): T 3 60-98 / 60-86, T 8 101-138 / 65-95, of the small layer 46 / 46. So 8
+// is where every layer is within a few percent of the better path; 3 to 7 tokens of the larger layers would gain up to 15 %
+// (a third with one context) by the mid-size path. Mid-size / prefill (128-row groups), picks: the first layer 1,024 809 /
+// 838, 1,600 861 / 865, 2,048 887 / 881, 4,096 952 / 915; the second 1,200 1,889 / 1,882, 2,046 2,022 / 1,981; the third
+// 1,026 1,240 / 1,280, 2,052 1,391 / 1,395, 3,072 1,411 / 1,401; the small one 1,360 112 / 123, 1,368 136 / 128, 2,048 150 /
+// 138. The split path (BMX_PATH_SPLIT) is never chosen here: the mid-size path alone is faster wherever the split path would
+// send a call to the MFMA kernels.
 static int resolve_path(int path, int T, int topk)
 {
     if (path == BMX_PATH_DECODE || path == BMX_PATH_PREFILL || path == BMX_PATH_MID || path == BMX_PATH_SPLIT)

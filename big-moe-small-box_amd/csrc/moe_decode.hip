@@ -524,20 +524,21 @@ __device__ __forceinline__ int ep_unit()
 {
     return (blockIdx.x * GV_WAVES + (threadIdx.x >> 6)) * UPW + ((threadIdx.x & 63) >> 4);
 }
-constexpr long EP_SMALL = 16384;              // launches with fewer units use UPW = 1
-// The gate / up epilogue's own line: a wave per unit costs four times the activations of 16 lanes per unit, which shows once
-// the units fill the SIMDs (11,088 units, four splits: 16.8 us against 14.4)
+constexpr long EP_SMALL = 16384;              // launches with fewer units use UPW = 1 (the down epilogues)
+// The gate / up epilogue's own line: a wave per unit starts four times the waves of 16 lanes per unit, which spreads a small
+// launch over more CUs and costs once the units fill the SIMDs. Layer us, a wave / 16 lanes per unit: 64 experts of H
+// 2048, I 768, 384 units 62.7 / 65.2, 1,920 units 90.5 / 92.6, 3,696 units 97.9 / 99.2, 4,608 units 100.3 / 100.8, 6,144
+// units 104.9 / 104.6; 288 of H 4096, I 1536, 3,456 units 493 / 492, 4,320 units 557 / 548. The kernel alone at 11,088 units:
+// 16.8 / 14.4.
 constexpr long EP_SMALL_GU = 4096;
 static bool gu_grouped(long units) { return units < EP_SMALL_GU; }
 
 // gate / up epilogue: sum of the splits in split order -> fp16 gate / up (the stored GEMV / GEMM results) -> H128 * R * svh
 // -> activation -> * down suh -> H128 * R -> fp16 down-input row (exllamav3 kernel A epilogue order,
 // engine/kernels/x16/x16_dev.cu:245-283)
-template <int UPW>
 __global__ __launch_bounds__(GV_THREADS) void k_gu_epi(GvArgs a)
 {
-    if (UPW == 1 && (threadIdx.x & 63) >= 16) return;
-    const int u = ep_unit<UPW>(), j = threadIdx.x & 15;
+    const int u = ep_unit<4>(), j = threadIdx.x & 15;
     const int r = u / a.NB, cb = u % a.NB;
     if (r >= a.offsets[a.NE]) return;
     const int e = a.row_expert[r];
@@ -987,7 +988,7 @@ int launch_epilogue(const GvArgs& a, int stage, hipStream_t s)
     {
         case BMX_STAGE_ACT:
             if (gu_grouped(gu)) hipLaunchKernelGGL(k_gu_epi_w, wgs(gu, 1), dim3(GV_THREADS), 0, s, a);
-            else hipLaunchKernelGGL(k_gu_epi<4>, wgs(gu, 4), dim3(GV_THREADS), 0, s, a);
+            else hipLaunchKernelGGL(k_gu_epi, wgs(gu, 4), dim3(GV_THREADS), 0, s, a);
             break;
         case BMX_STAGE_COMBINE:
             if (cmb >= EP_SMALL) hipLaunchKernelGGL(k_dn_combine, wgs(cmb, 4), dim3(GV_THREADS), 0, s, a);
@@ -1238,14 +1239,14 @@ int decode_rows_per_group(int T) { return rows_per_group_of(T); }
 
 // ---- split path ---------------------------------------------------------------------------------------------------------
 // The mid-size MFMA kernel decodes an expert once per 32 rows and multiplies on MFMA; the GEMV decodes once per group of
-// up to 8 rows and pays an fdot2 per row and weight, but has the shorter start. Measured on the 16-token speculative-
-// verify batch (the DeepSeek shape, 4-6 rows per expert): GEMV 172.6, mid-size 128.6 us; on the GLM shape at 8 tokens
-// (1.5 rows per expert): GEMV 225.7, mid-size 293. Mixing the two per expert in one call runs both kernels back to back
-// and measured worse than either alone (151-168 us, 255-278 us), so the choice is per call: all experts on the
-// mid-size kernel when the call averages at least BMX_SPLIT_RATIO rows per unique expert (default 2.5), else all on the
-// GEMV; BMX_SPLIT_MIN_ROWS = n also sends experts with at least n rows to the mid-size kernel in a GEMV call (off by
-// default: on the GEMV-chosen calls measured, 16- and 32-token batches of both shapes, it only added the idle cost of
-// walking the units).
+// up to 8 rows and pays an fdot2 per row and weight, but has the shorter start. Layer us, GEMV / mid-size, H 4096: 16
+// tokens of one context (9 experts, 10.7 rows each, I 2048) 163 / 83; 8 tokens with picks spread (62 experts, 1.03 rows,
+// I 1536) 227 / 200, 2 tokens 76 / 84. Mixing the two per expert in one call runs both kernels back to back and measured
+// worse than either alone (128 and 244 us for the first two), so the choice is per call: all experts on the mid-size kernel
+// when the call averages at least BMX_SPLIT_RATIO rows per unique expert (default 2.5), else all on the GEMV;
+// BMX_SPLIT_MIN_ROWS = n also sends experts with at least n rows to the mid-size kernel in a GEMV call (off by default).
+// The ratio dates from a slower mid-size kernel: where this path keeps a call of spread picks on the GEMV, the mid-size path
+// itself is now faster from about 4 tokens on.
 int split_min_rows()
 {
     const char* v = getenv("BMX_SPLIT_MIN_ROWS");
