@@ -61,7 +61,7 @@ struct DecodePlan {
     int KS_gu, KS_dn, NB, NBH, G_max, R_max;
     size_t part_gu_bytes, part_dn_bytes, counters;
 };
-// The rules that take more k-splits than fill the chip at first (several-token GEMV calls; mid-size calls of few rows or few
+// The rules that take more k-splits than the plain plans (several-token GEMV calls; mid-size calls of small partials or few
 // waves) cost workspace. They apply while the call's partial sums and rows stay within this, so that no call outgrows
 // bmx_moe_layer_scratch by them; extra = false is the plan without them.
 constexpr size_t EXTRA_SPLITS_WS = BMX_SCRATCH_BYTES / 4 * 3;
